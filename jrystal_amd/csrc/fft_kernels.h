@@ -31,6 +31,7 @@ struct BoxGeom {
   const int* row_g0;    // [nrows+1] first mask point of each row
   const int* g_row;     // [ng]      row of each mask point
   const int* rowidx;    // [nxa][ny] row of (active plane, y), or -1
+  int mmax;             // largest |integer frequency| of a mask point
 };
 
 // y = scale * DFT_axis(x) along one axis of a (B, n0, n1, n2) complex box.
@@ -119,10 +120,11 @@ int launch_xline_vpsi64(double2* T, const double* v, int groups, int nstates,
                         const BoxGeom& geo, const double2* tw64,
                         hipStream_t s);
 
-// Row-buffer path (rowfft.hip) for cubic 64^3 and 128^3 boxes whose mask
-// spans at most 64 x-planes.  R[c][z][row] (row stride geo.rstride) holds
+// Row-buffer path (rowfft.hip) for cubic boxes: 64^3 and 128^3 with masks of
+// at most 64 x-planes, the other 7-smooth sides of 32 to 80 with alias-free
+// masks (|m| <= n / 4).  R[c][z][row] (row stride geo.rstride) holds
 // the z-transformed rows of chunk state c; densities and potentials on
-// this path are z-major, [z][y][x].  tw is the length-n twiddle table.
+// this path are z-major, [z][x][y].  tw is the length-n twiddle table.
 bool use_rowpath(const BoxGeom& geo);
 // Row blocks of the row passes (the gather writes that many kinetic and
 // band-energy partials per state).
@@ -131,13 +133,13 @@ int row_chunks(const BoxGeom& geo);
 int zplane_groups(const BoxGeom& geo, int nstates);
 int launch_row_ifft(const double2* q, double2* R, int64_t state0, int nstates,
                     const BoxGeom& geo, const double2* tw, hipStream_t s);
-// rho_part[g][z][y][x] += sum_{c in group g} occ |psi_c|^2 / vol, or =
+// rho_part[g][z][x][y] += sum_{c in group g} occ |psi_c|^2 / vol, or =
 // with store (then every group's plane is written, empty groups with zeros)
 int launch_zplane_density(const double2* R, double* rho_part, int groups,
                           const double* occ, int64_t state0, int nstates,
                           double inv_vol, const BoxGeom& geo,
                           const double2* tw, bool store, hipStream_t s);
-// R[c] <- rows of FFT_xy(v * IFFT_xy(R[c])) (in place), v [z][y][x]
+// R[c] <- rows of FFT_xy(v * IFFT_xy(R[c])) (in place), v [z][x][y]
 int launch_zplane_vpsi(double2* R, const double* v, int groups, int nstates,
                        const BoxGeom& geo, const double2* tw, hipStream_t s);
 // qbar and kinetic partials kin_partial[st * row_chunks + chunk]
@@ -145,9 +147,10 @@ int launch_row_fft_gather(const double2* R, const double2* q, double2* qbar,
                           double* kin_partial, int64_t state0, int nstates,
                           const BoxGeom& geo, const double2* tw,
                           const GatherParams& gp, hipStream_t s);
-// [ns][z][y][x] -> [ns][x][y][z] for cubic n^3 boxes.
-int launch_zmajor_to_xmajor(const double* in, double* out, int ns, int n,
-                            hipStream_t s);
+// out[s][c][r] = in[s][r][c] for ns matrices of nr x nc: [z][x][y] ->
+// [x][y][z] with (nr, nc) = (nz, nx ny), and back with (nx ny, nz).
+int launch_rotate_axes(const double* in, double* out, int ns, int nr, int nc,
+                       hipStream_t s);
 
 // Largest plane (ny*nz) the fused plane kernels hold in LDS.
 constexpr int kPlaneCap = 6400;

@@ -136,7 +136,7 @@ struct jrx_plan {
   int xc = JRX_XC_LDA_X;    // JRX_XC_* terms
   bool rowpath = false;     // row-buffer FFT path (z-major rho and v)
   int row_chunks = 0;       // row blocks of the row passes
-  CellParams cpz;           // the cell with box axes (z, y, x)
+  CellParams cpz;           // the cell with box axes (z, x, y)
   GramSplit gsw, gsq;
   int kin_parts_max = 0, rec_parts = 0;
   // timing
@@ -285,6 +285,9 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->geo.nx = nx; p->geo.ny = ny; p->geo.nz = nz; p->geo.ng = ng;
   p->geo.nxa = (int)plane_x.size();
   p->geo.max_rows = max_rows;
+  p->geo.mmax = 0;
+  for (short m : g_m)
+    if (abs(m) > p->geo.mmax) p->geo.mmax = abs(m);
   int rc;
   int* tmp = nullptr;
   if ((rc = upload(p, plane_g0.data(), plane_g0.size(), &tmp))) return rc;
@@ -325,7 +328,7 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->cp.natom = d->natom;
   p->cp.pos = dpos;
   p->cp.charge = dchg;
-  // FFT path: the row buffer for cubic 64^3 / 128^3 boxes (fft_variant 0),
+  // FFT path: the row buffer for the cubic boxes it covers (fft_variant 0),
   // else the plane buffer (register 64-point kernels where they apply, or
   // the runtime-radix kernels everywhere with fft_variant 1).
   // JRX_FFT_GENERIC=1 selects the runtime-radix kernels too (cross-checks).
@@ -344,7 +347,7 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   JRX_CHECK_HIP(hipDeviceGetAttribute(
       &max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, p->device));
   const int nb = d->nb;
-  // (the row path's largest block holds an nz x 72 z-plane and twiddles)
+  // (the row path's largest block holds an nz x 73 z-plane)
   const size_t lds_plane =
       (p->rowpath ? (size_t)nz * 73 : (size_t)ny * nz) * sizeof(double2);
   // (the output transpose of jrx_plan_orthonormal_params: [nb][65])
@@ -396,13 +399,15 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->groups = p->rowpath ? zplane_groups(p->geo, sweep_states)
                          : xline_groups(p->geo, sweep_states, p->xline_blocks);
   p->row_chunks = p->rowpath ? row_chunks(p->geo) : 0;
-  // z-major cell of the row path: box axes (z, y, x)
+  // z-major cell of the row path: box axes (z, x, y)
   p->cpz = p->cp;
   p->cpz.nx = nz;
-  p->cpz.nz = nx;
+  p->cpz.ny = nx;
+  p->cpz.nz = ny;
   for (int i = 0; i < 3; ++i) {
     p->cpz.B[i] = p->B[6 + i];
-    p->cpz.B[6 + i] = p->B[i];
+    p->cpz.B[3 + i] = p->B[i];
+    p->cpz.B[6 + i] = p->B[3 + i];
   }
   // The geometry-only factor of the external term, S(G) / (|G|^2 + 1e-10),
   // on the box rho lives in (it does not change between evaluations).
@@ -1103,7 +1108,7 @@ static int timing_end(jrx_plan* p, hipStream_t s, int slot, int cls) {
 
 // v = dE/drho of rho (Hartree + external + xc, the vol/N weight included),
 // both in the plan's layout (z-major on the row path, whose box axes are
-// (z, y, x)).  The Hartree/external partials go to the workspace's eh/ee
+// (z, x, y)).  The Hartree/external partials go to the workspace's eh/ee
 // (*nrec of them) and the xc partials to exc (*nexc).  ks: the Kohn-Sham
 // effective potential of the band driver, which differs from dE/drho only
 // in the spin-polarised LDA exchange term.
@@ -1119,17 +1124,18 @@ static int potential_stage(jrx_plan* p, double* rho, double* v, char* ws,
   double* exc = dptr(p->o_exc);
   const CellParams& cpb = p->rowpath ? p->cpz : p->cp;
   const FftLen& L0 = p->rowpath ? p->Lz : p->Lx;
-  const FftLen& L2 = p->rowpath ? p->Lx : p->Lz;
+  const FftLen& L1 = p->rowpath ? p->Lx : p->Ly;
+  const FftLen& L2 = p->rowpath ? p->Ly : p->Lz;
   JRX_T(JRX_K_POTENTIAL, fft3d_real_forward(rho, p->ns, box, cpb.nx, cpb.ny,
-                                            cpb.nz, L0, p->Ly, L2, s));
+                                            cpb.nz, L0, L1, L2, s));
   double2* gb = p->o_gb ? cptr(p->o_gb) : nullptr;
   if (gb)  // density gradients of the GGA terms, from fftn(rho)
     JRX_T(JRX_K_POTENTIAL,
-          xc_stage_gradients(box, gb, cpb, L0, p->Ly, L2, s));
+          xc_stage_gradients(box, gb, cpb, L0, L1, L2, s));
   JRX_T(JRX_K_POTENTIAL,
         launch_potential_rec(box, box, eh, ee, cpb, nrec, s, p->d_sterm));
   JRX_T(JRX_K_POTENTIAL, fft3d(box, box, 1, cpb.nx, cpb.ny, cpb.nz, true,
-                               1.0 / (double)p->N, L0, p->Ly, L2, s));
+                               1.0 / (double)p->N, L0, L1, L2, s));
   if (p->xc == JRX_XC_LDA_X)
     JRX_T(JRX_K_POTENTIAL, launch_potential_real(box, rho, v, exc, p->ns,
                                                  p->N, p->vol, p->cx, nexc,
@@ -1137,7 +1143,7 @@ static int potential_stage(jrx_plan* p, double* rho, double* v, char* ws,
   else
     JRX_T(JRX_K_POTENTIAL,
           xc_stage_potential(box, rho, v, gb, exc, nexc, cpb, p->xc, L0,
-                             p->Ly, L2, s));
+                             L1, L2, s));
   return JRX_OK;
 }
 
@@ -1375,7 +1381,7 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
     JRX_T(JRX_K_OTHER, launch_nonlocal_finalize(p->d_enl, p->d_occ, S,
                                                 energies, s));
   if (rho_out && p->rowpath) {
-    if ((rc = launch_zmajor_to_xmajor(rho, rho_out, p->ns, p->nx, s)))
+    if ((rc = launch_rotate_axes(rho, rho_out, p->ns, p->nz, p->nx * p->ny, s)))
       return rc;
   } else if (rho_out) {
     JRX_CHECK_HIP(hipMemcpyAsync(rho_out, rho,
@@ -1440,9 +1446,9 @@ int jrx_plan_set_fixed_density(jrx_plan* p, const double* rho,
   double* r = reinterpret_cast<double*>(ws + p->o_rho);
   int rc;
   if (p->rowpath) {
-    // (x, y, z) -> the row path's (z, y, x): on its cubic box the axis swap
-    // is its own inverse
-    if ((rc = launch_zmajor_to_xmajor(rho, r, p->ns, p->nx, s))) return rc;
+    // (x, y, z) -> the row path's (z, x, y)
+    if ((rc = launch_rotate_axes(rho, r, p->ns, p->nx * p->ny, p->nz, s)))
+      return rc;
   } else {
     JRX_CHECK_HIP(hipMemcpyAsync(r, rho, bytes, hipMemcpyDeviceToDevice, s));
   }
@@ -1493,8 +1499,7 @@ __global__ void vloc_to_sterm_kernel(const double2* __restrict__ v,
   int64_t src = i;
   if (zmajor) {
     const int64_t a = i / ((int64_t)n * n), rem = i - a * n * n;
-    const int64_t b = rem / n, c = rem - b * n;  // i = (a, b, c) = (z, y, x)
-    src = (c * n + b) * n + a;
+    src = rem * n + a;  // i = (a, rem) = (z, (x, y))
   }
   const double2 t = v[src];
   sterm[i] = make_double2(t.x * scale, -t.y * scale);

@@ -1,0 +1,121 @@
+"""The row-buffer path at every box side it covers: energies, density,
+gradient and band energies against the runtime-radix plane kernels (another
+algorithm and other code), for masks that reach the edge of the alias-free
+window, stay one inside it, or have holes; masks beyond the window keep the
+plane path."""
+import numpy as np
+import pytest
+import torch
+
+from jrystal_amd.objective import EnergyPlan
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (32, 35, 36, 40, 42, 45, 48, 49, 50, 54, 56, 60, 63, 64, 70, 72, 75,
+         80)
+
+
+def _freq(n):
+  m = np.arange(n)
+  return np.where(m < (n + 1) // 2, m, m - n)
+
+
+def _mask(n, q, holes=0.0, seed=0):
+  """Ball of integer radius q (so that |m| = q occurs on every axis), with
+  a fraction of its points, whole rows and whole planes taken out."""
+  f = _freq(n).astype(float)
+  r2 = f[:, None, None]**2 + f[:, None]**2 + f**2
+  mask = r2 <= q * q
+  if holes:
+    rng = np.random.default_rng(seed)
+    mask &= rng.random(mask.shape) > holes
+    mask[_freq(n) == 2] = False
+    mask[:, _freq(n) == -1, :] &= rng.random((n, 1, n)) > 0.7
+    mask[0, 0, 0] = True
+  return mask
+
+
+def _run(n, mask, nk, nb, band, **opt):
+  cell = np.array([[6.1, 0.3, 0.0], [0.0, 5.7, -0.4], [0.2, 0.0, 6.6]])
+  pos = np.array([[0.1, 0.2, 0.3], [2.5, 2.9, 3.1]])
+  kpts = np.array([[0.0, 0.0, 0.0], [0.21, -0.13, 0.05]])[:nk]
+  occ = np.linspace(2.0, 0.5, nk * nb).reshape(1, nk, nb)
+  plan = EnergyPlan(pos, np.array([4.0, 3.0]), cell, mask, kpts, occ, **opt)
+  plan.set_band_energies(band)
+  gen = torch.Generator(device="cuda").manual_seed(n)
+  w = [torch.randn(plan.param_shape, generator=gen, device="cuda",
+                   dtype=torch.float64) for _ in range(2)]
+  r = plan.evaluate(*w, grad=True, density=True)
+  out = [r["energies"], r["dw_re"], r["dw_im"], r["density"]]
+  if band:
+    out.append(plan.band_energies())
+  path = plan.row_path
+  out = [x.cpu() for x in out]
+  plan.close()
+  return path, out
+
+
+def _close(a, b):
+  # two FP64 transforms of the same box: differences of a few rounding errors
+  # per radix stage (about 1e-15 each), amplified by the QR of random W by
+  # its condition number, below 10
+  for x, y in zip(a, b):
+    assert torch.linalg.norm(x - y) <= 2e-13 * torch.linalg.norm(y)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_row_sizes_match_plane_kernels(n):
+  for q, nk, nb, holes in ((n // 4, 1, 3, 0.0), (n // 4 - 1, 2, 5, 0.0),
+                           (n // 4, 2, 1, 0.2)):
+    mask = _mask(n, q, holes, seed=n)
+    print(f"n={n} q={q} holes={holes}", flush=True)
+    path, a = _run(n, mask, nk, nb, band=holes > 0)
+    assert path
+    ref, b = _run(n, mask, nk, nb, band=holes > 0, fft_variant=1)
+    assert not ref
+    _close(a, b)
+
+
+@pytest.mark.parametrize("n", (32, 45, 80))
+def test_wider_masks_keep_the_plane_path(n):
+  path, a = _run(n, _mask(n, n // 4 + 1), 1, 2, band=False)
+  assert not path
+  _, b = _run(n, _mask(n, n // 4 + 1), 1, 2, band=False, fft_variant=1)
+  _close(a, b)
+
+
+def test_row_path_64_wide_mask_with_holes():
+  mask = _mask(64, 21, 0.1, seed=3)
+  path, a = _run(64, mask, 2, 3, band=True)
+  assert path
+  _, b = _run(64, mask, 2, 3, band=True, fft_variant=1)
+  _close(a, b)
+
+
+def test_row_path_128_mask_beyond_the_window():
+  """A 128^3 mask with |m| = 40 along z and y and few x-planes (the kernels
+  without a window) against the oracle."""
+  from oracle import adjoint as OA
+  from oracle import grid as OG
+  n = 128
+  f = _freq(n).astype(float)
+  r2 = (f[:, None, None] / 9)**2 + (f[:, None] / 40)**2 + (f / 40)**2
+  mask = r2 <= 1.0
+  cell = 9.0 * np.eye(3)
+  pos = np.array([[0.5, 0.4, 0.3]])
+  kpts = np.zeros((1, 3))
+  occ = np.array([[[2.0, 1.0]]])
+  plan = EnergyPlan(pos, np.array([3.0]), cell, mask, kpts, occ)
+  assert plan.row_path
+  rng = np.random.default_rng(5)
+  p = {k: rng.standard_normal(plan.param_shape) for k in ("w_re", "w_im")}
+  r = plan.evaluate(p["w_re"], p["w_im"], grad=True, density=True)
+  prob = OA.Problem(mask=mask, g_vector_grid=OG.g_vectors(cell, [n] * 3),
+                    kpts=kpts, vol=float(np.linalg.det(cell)),
+                    occupation=occ, positions=pos, charges=np.array([3.0]))
+  parts, grad, rho = OA.energy_and_grad(p, prob)
+  assert abs(float(r["energies"][4]) - parts["total"]) < 1e-8
+  assert np.max(np.abs(r["density"].cpu().numpy() - rho)) < 1e-10
+  for k in ("w_re", "w_im"):
+    g = r["d" + k].cpu().numpy()
+    assert np.max(np.abs(g - grad[k])) < 1e-7 * np.max(np.abs(grad[k]))

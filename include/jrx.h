@@ -77,8 +77,9 @@ typedef struct {
   const double* occupation;/* host [ns*nk*nb]                               */
   int xc;                  /* JRX_XC_* terms OR-ed; 0 = lda_x              */
   int chunk_states;        /* states per FFT chunk, 0 = automatic           */
-  int fft_variant;         /* 0 = automatic (row buffer for cubic 64^3 and
-                              128^3 boxes, else plane buffer), 1 = plane
+  int fft_variant;         /* 0 = automatic (row buffer for the boxes it
+                              covers, jrx_plan_info.row_path, else plane
+                              buffer), 1 = plane
                               buffer with runtime-radix kernels only, 2 =
                               plane buffer (register 64-point kernels where
                               they apply)                                   */
@@ -101,7 +102,10 @@ typedef struct {
   int chunk_states;   /* states per FFT chunk                               */
   int keep_planes;    /* 1: the adjoint sweep reuses the forward planes     */
   size_t workspace_bytes;
-  int row_path;       /* 1: row-buffer FFT path (cubic 64^3 / 128^3 boxes)  */
+  int row_path;       /* 1: row-buffer FFT path: nx = ny among the 7-smooth
+                         sides of 32 to 80 (z: to 126), mask frequencies at
+                         most n / 4; 64 and 128: any mask of at most 64
+                         x-planes                                           */
   int rows;           /* (x, y) lines along z that hold mask points         */
 } jrx_plan_info;
 int jrx_plan_get_info(const jrx_plan* plan, jrx_plan_info* info);

@@ -31,7 +31,8 @@ struct BoxGeom {
   const int* row_g0;    // [nrows+1] first mask point of each row
   const int* g_row;     // [ng]      row of each mask point
   const int* rowidx;    // [nxa][ny] row of (active plane, y), or -1
-  int mmax;             // largest |integer frequency| of a mask point
+  int mmax_xy, mmax_z;  // largest |integer frequency| of a mask point along
+                        // x and y, and along z
 };
 
 // y = scale * DFT_axis(x) along one axis of a (B, n0, n1, n2) complex box.
@@ -120,11 +121,12 @@ int launch_xline_vpsi64(double2* T, const double* v, int groups, int nstates,
                         const BoxGeom& geo, const double2* tw64,
                         hipStream_t s);
 
-// Row-buffer path (rowfft.hip) for cubic boxes: 64^3 and 128^3 with masks of
-// at most 64 x-planes, the other 7-smooth sides of 32 to 80 with alias-free
-// masks (|m| <= n / 4).  R[c][z][row] (row stride geo.rstride) holds
-// the z-transformed rows of chunk state c; densities and potentials on
-// this path are z-major, [z][x][y].  tw is the length-n twiddle table.
+// Row-buffer path (rowfft.hip) for boxes with nx = ny: 64^3 and 128^3 with
+// masks of at most 64 x-planes, the other 7-smooth sides of 32 to 80 (z: to
+// 126) with alias-free masks (|m| <= n / 4).  R[c][z][row] (row stride
+// geo.rstride) holds the z-transformed rows of chunk state c; densities and
+// potentials on this path are z-major, [z][x][y].  tw is the twiddle table
+// of nz (row passes) or nx (z-plane passes).
 bool use_rowpath(const BoxGeom& geo);
 // Row blocks of the row passes (the gather writes that many kinetic and
 // band-energy partials per state).

@@ -285,9 +285,11 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->geo.nx = nx; p->geo.ny = ny; p->geo.nz = nz; p->geo.ng = ng;
   p->geo.nxa = (int)plane_x.size();
   p->geo.max_rows = max_rows;
-  p->geo.mmax = 0;
-  for (short m : g_m)
-    if (abs(m) > p->geo.mmax) p->geo.mmax = abs(m);
+  p->geo.mmax_xy = p->geo.mmax_z = 0;
+  for (size_t i = 0; i < g_m.size(); ++i) {
+    int& most = i % 3 == 2 ? p->geo.mmax_z : p->geo.mmax_xy;
+    if (abs(g_m[i]) > most) most = abs(g_m[i]);
+  }
   int rc;
   int* tmp = nullptr;
   if ((rc = upload(p, plane_g0.data(), plane_g0.size(), &tmp))) return rc;
@@ -328,7 +330,7 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->cp.natom = d->natom;
   p->cp.pos = dpos;
   p->cp.charge = dchg;
-  // FFT path: the row buffer for the cubic boxes it covers (fft_variant 0),
+  // FFT path: the row buffer for the boxes it covers (fft_variant 0),
   // else the plane buffer (register 64-point kernels where they apply, or
   // the runtime-radix kernels everywhere with fft_variant 1).
   // JRX_FFT_GENERIC=1 selects the runtime-radix kernels too (cross-checks).
@@ -347,9 +349,9 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   JRX_CHECK_HIP(hipDeviceGetAttribute(
       &max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, p->device));
   const int nb = d->nb;
-  // (the row path's largest block holds an nz x 73 z-plane)
+  // (the row path's largest block holds less than nx rows of 73)
   const size_t lds_plane =
-      (p->rowpath ? (size_t)nz * 73 : (size_t)ny * nz) * sizeof(double2);
+      (p->rowpath ? (size_t)nx * 73 : (size_t)ny * nz) * sizeof(double2);
   // (the output transpose of jrx_plan_orthonormal_params: [nb][65])
   const size_t lds_params = (size_t)nb * 65 * sizeof(double2);
   size_t need = lds_plane;
@@ -1256,7 +1258,7 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
         double2* Tc = p->keep_planes ? T + st0 * plane_elems : T;
         if (p->rowpath) {
           JRX_T(JRX_K_PLANE_IFFT,
-                launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lx.tw, s));
+                launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lz.tw, s));
           JRX_T(JRX_K_XLINE_DENSITY,
                 launch_zplane_density(Tc, rpart, zplane_groups(p->geo, nst),
                                       p->d_occ, st0, nst, 1.0 / p->vol,
@@ -1310,14 +1312,14 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
         if (p->rowpath) {
           if (!planes_ready)
             JRX_T(JRX_K_PLANE_IFFT,
-                  launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lx.tw, s));
+                  launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lz.tw, s));
           JRX_T(JRX_K_XLINE_VPSI,
                 launch_zplane_vpsi(Tc, vv + sp * p->N,
                                    zplane_groups(p->geo, nst), nst, p->geo,
                                    p->Lx.tw, s));
           JRX_T(JRX_K_PLANE_FFT_GATHER,
                 launch_row_fft_gather(Tc, q, qbar, kin, st0, nst, p->geo,
-                                      p->Lx.tw, gp, s));
+                                      p->Lz.tw, gp, s));
         } else if (reg64) {
           if (!planes_ready)
             JRX_T(JRX_K_PLANE_IFFT, launch_plane_ifft64(q, Tc, st0, nst,
@@ -1490,16 +1492,16 @@ int jrx_plan_subspace_hamiltonian(const jrx_plan* p, double* h,
 }
 
 // sterm[i] = conj(v[x-major index of i]) * scale on the plan's box (on the
-// row path the box axes are (z, y, x) of a cubic n^3 box).
+// row path the box axes are (z, x, y)).
 __global__ void vloc_to_sterm_kernel(const double2* __restrict__ v,
                                      double2* __restrict__ sterm, int64_t N,
-                                     int n, int zmajor, double scale) {
+                                     int nz, int zmajor, double scale) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   int64_t src = i;
   if (zmajor) {
-    const int64_t a = i / ((int64_t)n * n), rem = i - a * n * n;
-    src = rem * n + a;  // i = (a, rem) = (z, (x, y))
+    const int64_t nxy = N / nz, z = i / nxy;
+    src = (i - z * nxy) * nz + z;  // i = (z, (x, y))
   }
   const double2 t = v[src];
   sterm[i] = make_double2(t.x * scale, -t.y * scale);
@@ -1535,7 +1537,7 @@ int jrx_plan_set_external_potential(jrx_plan* p, const double* v_rec,
   const double scale = -p->vol / (4.0 * M_PI * (double)p->N);
   hipLaunchKernelGGL(vloc_to_sterm_kernel, dim3(ceil_div(p->N, 256)),
                      dim3(256), 0, s, reinterpret_cast<const double2*>(v_rec),
-                     p->d_sterm, p->N, p->nx, p->rowpath ? 1 : 0, scale);
+                     p->d_sterm, p->N, p->nz, p->rowpath ? 1 : 0, scale);
   JRX_LAUNCH_CHECK();
   p->custom_vloc = true;
   return JRX_OK;

@@ -236,7 +236,7 @@ struct RDft<16, INV> {
 // stage.  XS, A, B: exchange slots through LDS, value (a, j) of a line at
 // a A + j B of the line's XS doubles, the layout with the fewest bank
 // conflicts of the transform's writes and reads (16 lanes per cycle on 32
-// banks, counted over all A, B and XS up to 1.35 N; at 75 points 45 extra
+// banks, counted over all A, B and XS up to 1.35 N + 8; at 75 points 45 extra
 // cycles for 120, against 90 with a L + j).
 template <int N>
 struct LineSplit;
@@ -264,6 +264,18 @@ JRX_LINE_SPLIT(72, 12, 6, 83, 1, 14)
 JRX_LINE_SPLIT(75, 15, 5, 87, 5, 4)
 JRX_LINE_SPLIT(80, 10, 8, 0, 0, 0)
 JRX_LINE_SPLIT(128, 16, 8, 0, 0, 0)
+// (z axes only: the row passes)
+JRX_LINE_SPLIT(81, 9, 9, 87, 1, 9)
+JRX_LINE_SPLIT(84, 12, 7, 101, 2, 13)
+JRX_LINE_SPLIT(90, 15, 6, 117, 7, 2)
+JRX_LINE_SPLIT(96, 12, 8, 0, 0, 0)
+JRX_LINE_SPLIT(98, 14, 7, 121, 1, 17)
+JRX_LINE_SPLIT(100, 10, 10, 103, 1, 10)
+JRX_LINE_SPLIT(105, 15, 7, 121, 1, 17)
+JRX_LINE_SPLIT(108, 12, 9, 151, 1, 17)
+JRX_LINE_SPLIT(112, 14, 8, 0, 0, 0)
+JRX_LINE_SPLIT(120, 15, 8, 0, 0, 0)
+JRX_LINE_SPLIT(126, 14, 9, 151, 1, 17)
 #undef JRX_LINE_SPLIT
 
 // Lane-bit swaps of two registers: after it, a lane with the bit set holds

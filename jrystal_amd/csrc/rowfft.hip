@@ -1,5 +1,6 @@
-// Row-buffer path of the fused evaluation, for cubic boxes (sides of
-// JRX_ROW_SIZES, and 128).
+// Row-buffer path of the fused evaluation, for boxes with square (x, y)
+// planes (sides of JRX_Z_SIZES, 32, 64 and 128) and any of the JRX_ROW_SIZES
+// along z.
 //
 // A state's 3D transform runs through a row buffer R[state][z][row], where
 // the rows are the (x, y) lines along z that hold mask points (numbered in
@@ -20,26 +21,32 @@
 
 namespace jrx {
 
-// Sides with an alias-free window only; 64 and 128 also take wider masks.
-#define JRX_ROW_SIZES(X)                                                    \
+// Lengths with an alias-free window (PR 1) only; 32, 64 and 128 also have the
+// tighter one (PR 2), 64 and 128 kernels for any mask (PR 0).
+#define JRX_Z_SIZES(X)                                                      \
   X(35) X(36) X(40) X(42) X(45) X(48) X(49) X(50) X(54) X(56) X(60) X(63)   \
   X(70) X(72) X(75) X(80)
+#define JRX_ROW_SIZES(X)                                                    \
+  JRX_Z_SIZES(X)                                                            \
+  X(81) X(84) X(90) X(96) X(98) X(100) X(105) X(108) X(112) X(120) X(126)
 
-// Mask window of the box: 2 or 1 (see rowfft_kernels.h), 0 for any mask of
-// 64^3 and 128^3 boxes with at most 64 x-planes, -1 = no row path.
-static int row_window(const BoxGeom& geo) {
-  const int n = geo.nx;
-  if (geo.ny != n || geo.nz != n || geo.nxa > 64 || geo.nrows <= 0 ||
-      geo.nrows > 32767)
-    return -1;
-  const bool tight = geo.mmax <= n / 4 - 1, fits = geo.mmax <= n / 4;
+// Window of the largest |frequency| m along axes of n points (PR), -1 = none.
+static int window_of(int n, int m, bool row) {
+  const bool tight = m <= n / 4 - 1, fits = m <= n / 4;
   switch (n) {
     case 32:
       return tight ? 2 : fits ? 1 : -1;
     case 64:
+      return tight ? 2 : fits ? 1 : 0;
     case 128:
-      return tight ? 2 : (fits && n == 64) ? 1 : 0;
+      return tight ? 2 : 0;
 #define JRX_X(NN) case NN:
+    JRX_Z_SIZES(JRX_X)
+      return fits ? 1 : -1;
+    default:
+      break;
+  }
+  switch (row ? n : 0) {
     JRX_ROW_SIZES(JRX_X)
 #undef JRX_X
       return fits ? 1 : -1;
@@ -47,28 +54,53 @@ static int row_window(const BoxGeom& geo) {
       return -1;
   }
 }
+static int row_window(const BoxGeom& geo) {
+  return window_of(geo.nz, geo.mmax_z, true);
+}
+static int z_window(const BoxGeom& geo) {
+  return window_of(geo.nx, geo.mmax_xy, false);
+}
 
-bool use_rowpath(const BoxGeom& geo) { return row_window(geo) >= 0; }
+// Square planes, a window along every axis, and not beyond what the plane
+// path takes unless cubic.  (The z-plane passes hold the active columns of a
+// plane in LDS and row indices in 16 bits.)
+bool use_rowpath(const BoxGeom& geo) {
+  return geo.nx == geo.ny && geo.nxa <= 64 && geo.nrows > 0 &&
+         geo.nrows <= 32767 &&
+         (geo.nz == geo.nx || geo.ny * geo.nz <= kPlaneCap) &&
+         row_window(geo) >= 0 && z_window(geo) >= 0;
+}
 
-// CALL(N, PR) of the box's kernels.
+static int unsupported_box() {
+  set_error("row path: unsupported box");
+  return JRX_ERR_UNSUPPORTED;
+}
+
+// CALL(N, PR) of the box: z-plane passes, row passes.
+#define JRX_DISPATCH_COMMON(CALL)                                           \
+  case 32 * 4 + 1: return CALL(32, 1);                                      \
+  case 32 * 4 + 2: return CALL(32, 2);                                      \
+  case 64 * 4 + 0: return CALL(64, 0);                                      \
+  case 64 * 4 + 1: return CALL(64, 1);                                      \
+  case 64 * 4 + 2: return CALL(64, 2);                                      \
+  case 128 * 4 + 0: return CALL(128, 0);                                    \
+  case 128 * 4 + 2: return CALL(128, 2);
+#define JRX_Z_DISPATCH(CALL)                                                \
+  switch (geo.nx * 4 + z_window(geo)) {                                     \
+    JRX_DISPATCH_COMMON(CALL)                                               \
+    JRX_Z_SIZES(JRX_X)                                                      \
+    default: return unsupported_box();                                      \
+  }
 #define JRX_ROW_DISPATCH(CALL)                                              \
-  switch (geo.nx * 4 + row_window(geo)) {                                   \
-    case 32 * 4 + 1: return CALL(32, 1);                                    \
-    case 32 * 4 + 2: return CALL(32, 2);                                    \
-    case 64 * 4 + 0: return CALL(64, 0);                                    \
-    case 64 * 4 + 1: return CALL(64, 1);                                    \
-    case 64 * 4 + 2: return CALL(64, 2);                                    \
-    case 128 * 4 + 0: return CALL(128, 0);                                  \
-    case 128 * 4 + 2: return CALL(128, 2);                                  \
+  switch (geo.nz * 4 + row_window(geo)) {                                   \
+    JRX_DISPATCH_COMMON(CALL)                                               \
     JRX_ROW_SIZES(JRX_X)                                                    \
-    default:                                                                \
-      set_error("row path: unsupported box");                               \
-      return JRX_ERR_UNSUPPORTED;                                           \
+    default: return unsupported_box();                                      \
   }
 
 int row_chunks(const BoxGeom& geo) {
   int rpb = 0;
-  switch (geo.nx) {
+  switch (geo.nz) {
 #define JRX_X(NN) case NN: rpb = RowBlock<NN>::RPB; break;
     JRX_ROW_SIZES(JRX_X)
     JRX_X(32)
@@ -95,7 +127,7 @@ int zplane_groups(const BoxGeom& geo, int nstates) {
 
 int launch_row_ifft(const double2* q, double2* R, int64_t state0, int nstates,
                     const BoxGeom& geo, const double2* tw, hipStream_t s) {
-#define JRX_CALL(NN, PR) RowPath<NN, PR>::ifft(q, R, state0, nstates, geo, tw, s)
+#define JRX_CALL(NN, PR) RowPass<NN, PR>::ifft(q, R, state0, nstates, geo, tw, s)
 #define JRX_X(NN) case NN * 4 + 1: return JRX_CALL(NN, 1);
   JRX_ROW_DISPATCH(JRX_CALL)
 #undef JRX_X
@@ -107,7 +139,7 @@ int launch_row_fft_gather(const double2* R, const double2* q, double2* qbar,
                           const BoxGeom& geo, const double2* tw,
                           const GatherParams& gp, hipStream_t s) {
 #define JRX_CALL(NN, PR)                                                    \
-  RowPath<NN, PR>::gather(R, q, qbar, kin_partial, state0, nstates, geo, tw, \
+  RowPass<NN, PR>::gather(R, q, qbar, kin_partial, state0, nstates, geo, tw, \
                           gp, s)
 #define JRX_X(NN) case NN * 4 + 1: return JRX_CALL(NN, 1);
   JRX_ROW_DISPATCH(JRX_CALL)
@@ -120,19 +152,19 @@ int launch_zplane_density(const double2* R, double* rho_part, int groups,
                           double inv_vol, const BoxGeom& geo,
                           const double2* tw, bool store, hipStream_t s) {
 #define JRX_CALL(NN, PR)                                                    \
-  RowPath<NN, PR>::density(R, rho_part, groups, occ, state0, nstates,       \
+  ZPass<NN, PR>::density(R, rho_part, groups, occ, state0, nstates,       \
                            inv_vol, geo, tw, store, s)
 #define JRX_X(NN) case NN * 4 + 1: return JRX_CALL(NN, 1);
-  JRX_ROW_DISPATCH(JRX_CALL)
+  JRX_Z_DISPATCH(JRX_CALL)
 #undef JRX_X
 #undef JRX_CALL
 }
 
 int launch_zplane_vpsi(double2* R, const double* v, int groups, int nstates,
                        const BoxGeom& geo, const double2* tw, hipStream_t s) {
-#define JRX_CALL(NN, PR) RowPath<NN, PR>::vpsi(R, v, groups, nstates, geo, tw, s)
+#define JRX_CALL(NN, PR) ZPass<NN, PR>::vpsi(R, v, groups, nstates, geo, tw, s)
 #define JRX_X(NN) case NN * 4 + 1: return JRX_CALL(NN, 1);
-  JRX_ROW_DISPATCH(JRX_CALL)
+  JRX_Z_DISPATCH(JRX_CALL)
 #undef JRX_X
 #undef JRX_CALL
 }

@@ -1,11 +1,16 @@
-// Row-path kernels of some box sides (see rowfft_kernels.h).
+// Row-path kernels of some lengths (see rowfft_kernels.h).
 #define JRX_ROWFFT_KERNELS
 #include "rowfft_kernels.h"
 
 namespace jrx {
-template struct RowPath<60, 1>;
-template struct RowPath<63, 1>;
-template struct RowPath<64, 0>;
-template struct RowPath<64, 1>;
-template struct RowPath<64, 2>;
+template struct ZPass<60, 1>;
+template struct ZPass<63, 1>;
+template struct ZPass<64, 0>;
+template struct ZPass<64, 1>;
+template struct ZPass<64, 2>;
+template struct RowPass<60, 1>;
+template struct RowPass<63, 1>;
+template struct RowPass<64, 0>;
+template struct RowPass<64, 1>;
+template struct RowPass<64, 2>;
 }  // namespace jrx

@@ -1,9 +1,12 @@
-// Row-path kernels of some box sides (see rowfft_kernels.h).
+// Row-path kernels of some lengths (see rowfft_kernels.h).
 #define JRX_ROWFFT_KERNELS
 #include "rowfft_kernels.h"
 
 namespace jrx {
-template struct RowPath<80, 1>;
-template struct RowPath<128, 0>;
-template struct RowPath<128, 2>;
+template struct ZPass<80, 1>;
+template struct ZPass<128, 0>;
+template struct ZPass<128, 2>;
+template struct RowPass<80, 1>;
+template struct RowPass<128, 0>;
+template struct RowPass<128, 2>;
 }  // namespace jrx

@@ -1,8 +1,9 @@
-// Kernels of the row-buffer path (rowfft.hip), one set per box side N and
-// mask window PR:
-//   PR 1: every mask point has |m| <= N / 4 along every axis (a density box
-//         that is free of aliasing); PR 2: |m| <= N / 4 - 1; PR 0: any mask
-//         of at most 64 x-planes (N = 64 and 128 only).
+// Kernels of the row-buffer path (rowfft.hip): row passes, one set per length
+// N of the z axis, and z-plane passes, one set per side N of the square (x, y)
+// planes; each with the mask's window PR along the axes it transforms:
+//   PR 1: every mask point has |m| <= N / 4 (a density box that is free of
+//         aliasing); PR 2: |m| <= N / 4 - 1; PR 0: any mask (z-plane passes:
+//         of at most 64 x-planes; N = 64 and 128 only).
 // With a window, the first radix stage of an inverse transform has about half
 // of its inputs and the last one of a forward transform about half of its
 // outputs: the loads, stores and additions of the rest are not there.
@@ -15,13 +16,16 @@ namespace jrx {
 // Host launchers of one (N, PR); defined below, instantiated in
 // rowfft_*.hip.
 template <int N, int PR>
-struct RowPath {
+struct RowPass {
   static int ifft(const double2* q, double2* R, int64_t state0, int nstates,
                   const BoxGeom& geo, const double2* tw, hipStream_t s);
   static int gather(const double2* R, const double2* q, double2* qbar,
                     double* kin_partial, int64_t state0, int nstates,
                     const BoxGeom& geo, const double2* tw,
                     const GatherParams& gp, hipStream_t s);
+};
+template <int N, int PR>
+struct ZPass {
   static int density(const double2* R, double* rho_part, int groups,
                      const double* occ, int64_t state0, int nstates,
                      double inv_vol, const BoxGeom& geo, const double2* tw,
@@ -394,7 +398,7 @@ __global__ __launch_bounds__(NW * 64, 2) void zplane_density_kernel(
   const int G = gridDim.y, gi = blockIdx.y;
   const int per = (nstates + G - 1) / G;
   const int cb = gi * per, ce = min(nstates, cb + per);
-  double* part = rho_part + ((int64_t)gi * N + z) * N * N;  // [x][y]
+  double* part = rho_part + ((int64_t)gi * geo.nz + z) * N * N;  // [x][y]
   if (cb >= ce) {  // uniform over the block: an empty group
     if (store)
       for (int i = threadIdx.x; i < N * N; i += Z::NT) part[i] = 0.0;
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(NW * 64, 2) void zplane_density_kernel(
   for (int p = 0; p < YP; ++p)
 #pragma unroll
     for (int t = 0; t < Z::VP; ++t) acc[p][t] = 0.0;
-  const int64_t sstride = (int64_t)N * geo.rstride;
+  const int64_t sstride = (int64_t)geo.nz * geo.rstride;
   const double2* src0 = R + (int64_t)z * geo.rstride;
   double2 pre[Z::CP][Z::M];
   if constexpr (PF) zp.load(pre, src0 + (int64_t)cb * sstride);
@@ -480,7 +484,7 @@ __global__ __launch_bounds__(NW * 64, 2) void zplane_vpsi_kernel(
 #pragma unroll
     for (int p = 0; p < YP; ++p) load_v(vr[p], min(zp.line(p), N - 1));
   }
-  const int64_t sstride = (int64_t)N * geo.rstride;
+  const int64_t sstride = (int64_t)geo.nz * geo.rstride;
   double2* buf0 = R + (int64_t)z * geo.rstride;
   double2 pre[Z::CP][Z::M];
   if constexpr (PF) zp.load(pre, buf0 + (int64_t)cb * sstride);
@@ -548,7 +552,7 @@ __global__ __launch_bounds__(NW * 64, 2) void zplane_vpsi_kernel(
 
 // ------------------------------------------------------------ launchers --
 template <int N, int PR>
-int RowPath<N, PR>::ifft(const double2* q, double2* R, int64_t state0,
+int RowPass<N, PR>::ifft(const double2* q, double2* R, int64_t state0,
                          int nstates, const BoxGeom& geo, const double2* tw,
                          hipStream_t s) {
   constexpr int RPB = RowBlock<N>::RPB;
@@ -562,7 +566,7 @@ int RowPath<N, PR>::ifft(const double2* q, double2* R, int64_t state0,
 }
 
 template <int N, int PR>
-int RowPath<N, PR>::gather(const double2* R, const double2* q, double2* qbar,
+int RowPass<N, PR>::gather(const double2* R, const double2* q, double2* qbar,
                            double* kin_partial, int64_t state0, int nstates,
                            const BoxGeom& geo, const double2* tw,
                            const GatherParams& gp, hipStream_t s) {
@@ -588,7 +592,7 @@ struct ZWide {
 };
 
 template <int N, int PR>
-int RowPath<N, PR>::density(const double2* R, double* rho_part, int groups,
+int ZPass<N, PR>::density(const double2* R, double* rho_part, int groups,
                             const double* occ, int64_t state0, int nstates,
                             double inv_vol, const BoxGeom& geo,
                             const double2* tw, bool store, hipStream_t s) {
@@ -596,7 +600,7 @@ int RowPath<N, PR>::density(const double2* R, double* rho_part, int groups,
   constexpr int NW = ZWide<N, PR>::value ? 8 : S::NWD;
   constexpr bool PF = PR != 0 && S::PFD;
   hipLaunchKernelGGL((zplane_density_kernel<N, PR, NW, PF>),
-                     dim3(N, groups), dim3(NW * 64),
+                     dim3(geo.nz, groups), dim3(NW * 64),
                      (ZPlane<N, PR, NW>::kLds), s, R, rho_part, occ, state0,
                      nstates, inv_vol, geo, tw, store ? 1 : 0);
   JRX_LAUNCH_CHECK();
@@ -604,14 +608,14 @@ int RowPath<N, PR>::density(const double2* R, double* rho_part, int groups,
 }
 
 template <int N, int PR>
-int RowPath<N, PR>::vpsi(double2* R, const double* v, int groups, int nstates,
+int ZPass<N, PR>::vpsi(double2* R, const double* v, int groups, int nstates,
                          const BoxGeom& geo, const double2* tw,
                          hipStream_t s) {
   using S = ZShape<N>;
   constexpr int NW = ZWide<N, PR>::value ? 8 : S::NW;
   constexpr bool VR = S::VR, PF = PR != 0 && S::PFV;
   hipLaunchKernelGGL((zplane_vpsi_kernel<N, PR, NW, VR, PF>),
-                     dim3(N, groups), dim3(NW * 64),
+                     dim3(geo.nz, groups), dim3(NW * 64),
                      (ZPlane<N, PR, NW>::kLds), s, R, v, nstates, geo, tw);
   JRX_LAUNCH_CHECK();
   return JRX_OK;

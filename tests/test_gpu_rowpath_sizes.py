@@ -20,17 +20,19 @@ def _freq(n):
   return np.where(m < (n + 1) // 2, m, m - n)
 
 
-def _mask(n, q, holes=0.0, seed=0):
-  """Ball of integer radius q (so that |m| = q occurs on every axis), with
-  a fraction of its points, whole rows and whole planes taken out."""
-  f = _freq(n).astype(float)
-  r2 = f[:, None, None]**2 + f[:, None]**2 + f**2
-  mask = r2 <= q * q
+def _mask(n, q, holes=0.0, seed=0, nz=None, qz=None):
+  """Ball of integer radius q (so that |m| = q occurs on every axis; radius
+  qz along z), with a fraction of its points, whole rows and whole planes
+  taken out."""
+  nz, qz = nz or n, qz or q
+  f, fz = _freq(n) / q, _freq(nz) / qz
+  r2 = f[:, None, None]**2 + f[:, None]**2 + fz**2
+  mask = r2 <= 1.0 + 1e-12
   if holes:
     rng = np.random.default_rng(seed)
     mask &= rng.random(mask.shape) > holes
     mask[_freq(n) == 2] = False
-    mask[:, _freq(n) == -1, :] &= rng.random((n, 1, n)) > 0.7
+    mask[:, _freq(n) == -1, :] &= rng.random((n, 1, nz)) > 0.7
     mask[0, 0, 0] = True
   return mask
 
@@ -74,6 +76,44 @@ def test_row_sizes_match_plane_kernels(n):
     ref, b = _run(n, mask, nk, nb, band=holes > 0, fft_variant=1)
     assert not ref
     _close(a, b)
+
+
+@pytest.mark.parametrize("n,nz", [(32, z) for z in (
+  36, 64, 81, 84, 90, 96, 98, 100, 105, 108, 112, 120, 126, 128)] + [
+    (50, 35), (64, 45), (64, 100), (75, 32), (80, 64)])
+def test_square_plane_boxes_match_plane_kernels(n, nz):
+  for qz, holes in ((nz // 4, 0.0), (nz // 4 - 1, 0.2)):
+    mask = _mask(n, n // 4, holes, seed=nz, nz=nz, qz=qz)
+    print(f"n={n} nz={nz} qz={qz}", flush=True)
+    path, a = _run(n, mask, 2, 2, band=True)
+    assert path
+    ref, b = _run(n, mask, 2, 2, band=True, fft_variant=1)
+    assert not ref
+    _close(a, b)
+
+
+def test_fixed_density_and_local_potential_on_a_long_box():
+  """The axis rotations of the row path (band mode's density, a local
+  potential given on the box) on a non-cubic box."""
+  n, nz = 36, 45
+  mask = _mask(n, 9, nz=nz, qz=11)
+  rng = np.random.default_rng(2)
+  rho = rng.random((1, n, n, nz)) + 0.5
+  v = rng.standard_normal((n, n, nz)) + 1j * rng.standard_normal((n, n, nz))
+  res = []
+  for variant in (0, 1):
+    occ = np.ones((1, 1, 3))
+    plan = EnergyPlan(np.zeros((1, 3)), np.array([2.0]), 6.0 * np.eye(3),
+                      mask, np.zeros((1, 3)), occ, fft_variant=variant)
+    assert plan.row_path == (variant == 0)
+    plan.set_external_potential(v)
+    plan.set_fixed_density(rho)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    w = [torch.randn(plan.param_shape, generator=gen, device="cuda",
+                     dtype=torch.float64) for _ in range(2)]
+    r = plan.evaluate(*w, grad=True)
+    res.append([r[k].cpu() for k in ("energies", "dw_re", "dw_im")])
+  _close(*res)
 
 
 @pytest.mark.parametrize("n", (32, 45, 80))

@@ -124,16 +124,6 @@ int launch_potential_rec(const double2* rho_rec, double2* vrec,
   return JRX_OK;
 }
 
-// eps_x(n) = -cx n^(1/3) above the density threshold, else 0.
-__device__ __forceinline__ double lda_x_eps(double n, double cx) {
-  return n > 1e-15 ? -cx * cbrt(n) : 0.0;
-}
-__device__ __forceinline__ double lda_x_deps(double n, double cx) {
-  if (!(n > 1e-15)) return 0.0;
-  const double c = cbrt(n);
-  return -cx / (3.0 * c * c);
-}
-
 __global__ __launch_bounds__(kRedBlock) void potential_real_kernel(
     const double2* __restrict__ vbox, const double* __restrict__ rho,
     double* __restrict__ v, double* __restrict__ exc_part, int ns, int64_t N,
@@ -141,27 +131,8 @@ __global__ __launch_bounds__(kRedBlock) void potential_real_kernel(
   __shared__ double red[kRedBlock];
   const int64_t i = (int64_t)blockIdx.x * kRedBlock + threadIdx.x;
   double exc = 0.0;
-  if (i < N) {
-    const double w = vol / (double)N;
-    const double vhe = vbox[i].x;
-    if (ns == 1) {
-      const double r = rho[i];
-      const double e = lda_x_eps(r, cx);
-      exc = w * e * r;
-      v[i] = vhe + w * (4.0 / 3.0) * e;
-    } else {
-      // Spin-polarised exchange as in xc.py:56-59: eps = (e(2ru)+e(2rd))/2
-      // multiplies the total density.  v_s = d E / d rho_s = eps + rt
-      // d eps / d rho_s; the Kohn-Sham form (ks) of the band driver is
-      // vxc_lda (xc.py:109-124), eps + rho_s d eps / d rho_s.
-      const double ru = rho[i], rd = rho[N + i];
-      const double e = 0.5 * (lda_x_eps(2.0 * ru, cx) + lda_x_eps(2.0 * rd, cx));
-      const double rt = ru + rd;
-      exc = w * e * rt;
-      v[i] = vhe + w * (e + (ks ? ru : rt) * lda_x_deps(2.0 * ru, cx));
-      v[N + i] = vhe + w * (e + (ks ? rd : rt) * lda_x_deps(2.0 * rd, cx));
-    }
-  }
+  if (i < N)
+    exc = lda_x_point(vbox[i].x, rho, v, i, N, ns, vol / (double)N, cx, ks);
   const double t = block_sum(exc, red);
   if (threadIdx.x == 0) exc_part[blockIdx.x] = t;
 }

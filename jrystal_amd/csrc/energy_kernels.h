@@ -64,8 +64,20 @@ int launch_finalize_energies(const double* tb, const double* occ, int64_t S,
 
 int launch_fill(double* p, double v, int64_t n, hipStream_t s);
 
-// Exchange-correlation stage beyond LDA exchange (xc.hip), unpolarised.
 struct FftLen;
+// The whole potential stage of LDA exchange in three launches (boxfft.hip),
+// for boxes box_potential_size covers (two equal inner axes): (y, z) planes
+// of the real density; x lines forward, potential_rec, inverse; planes back
+// with potential_real at the points.  box is scratch; arguments and partials
+// as in the separate launchers (L12: the length of both inner axes).
+bool box_potential_size(const CellParams& cp);
+int box_potential_lda(const double* rho, double2* box, double* v, double* eh,
+                      double* ee, double* exc, int ns, double cx, bool ks,
+                      const CellParams& cp, const double2* sterm,
+                      const FftLen& L0, const FftLen& L12, int* nrec,
+                      int* nexc, hipStream_t s);
+
+// Exchange-correlation stage beyond LDA exchange (xc.hip), unpolarised.
 bool xc_is_gga(int flags);
 // gb[3][N] = ifftn(i G_d rho_rec) (the density gradient boxes; cp's box)
 // (gvec, optional: the G grid [N][3] to use instead of cp's basis)
@@ -81,6 +93,38 @@ int xc_stage_potential(const double2* vbox, const double* rho, double* v,
                        const CellParams& cp, int flags, const FftLen& L0,
                        const FftLen& L1, const FftLen& L2, hipStream_t s,
                        const double* gvec = nullptr);
+
+// eps_x(n) = -cx n^(1/3) above the density threshold, else 0.
+__device__ __forceinline__ double lda_x_eps(double n, double cx) {
+  return n > 1e-15 ? -cx * cbrt(n) : 0.0;
+}
+__device__ __forceinline__ double lda_x_deps(double n, double cx) {
+  if (!(n > 1e-15)) return 0.0;
+  const double c = cbrt(n);
+  return -cx / (3.0 * c * c);
+}
+// v at point i of N (all ns channels) from the Hartree + external potential
+// vhe there, and the point's exchange energy; w = vol / N.
+__device__ __forceinline__ double lda_x_point(
+    double vhe, const double* __restrict__ rho, double* __restrict__ v,
+    int64_t i, int64_t N, int ns, double w, double cx, int ks) {
+  if (ns == 1) {
+    const double r = rho[i];
+    const double e = lda_x_eps(r, cx);
+    v[i] = vhe + w * (4.0 / 3.0) * e;
+    return w * e * r;
+  }
+  // Spin-polarised exchange as in xc.py:56-59: eps = (e(2ru)+e(2rd))/2
+  // multiplies the total density.  v_s = d E / d rho_s = eps + rt
+  // d eps / d rho_s; the Kohn-Sham form (ks) of the band driver is
+  // vxc_lda (xc.py:109-124), eps + rho_s d eps / d rho_s.
+  const double ru = rho[i], rd = rho[N + i];
+  const double e = 0.5 * (lda_x_eps(2.0 * ru, cx) + lda_x_eps(2.0 * rd, cx));
+  const double rt = ru + rd;
+  v[i] = vhe + w * (e + (ks ? ru : rt) * lda_x_deps(2.0 * ru, cx));
+  v[N + i] = vhe + w * (e + (ks ? rd : rt) * lda_x_deps(2.0 * rd, cx));
+  return w * e * rt;
+}
 
 // Twiddle tables of the plan-less FFT entry points (a per-device cache).
 int cached_fftlen(int n, FftLen* L);

@@ -67,6 +67,15 @@ int launch_line_fft(const double2* in, double2* out, int64_t B, int n0, int n1,
                     int n2, int axis, bool inverse, double scale,
                     const FftLen& L, hipStream_t s, const double* rin,
                     int ns) {
+  if (!rin && box_line_size(L.n)) {
+    // register lines
+    const int64_t mid = (int64_t)n1 * n2;
+    if (axis == 2)
+      return box_line(in, out, 1, 0, B * n0 * n1, n2, 1, inverse, scale, L, s);
+    if (axis == 1)
+      return box_line(in, out, B * n0, mid, n2, 1, n2, inverse, scale, L, s);
+    return box_line(in, out, B, n0 * mid, mid, 1, mid, inverse, scale, L, s);
+  }
   if (rin && (axis != 2 || inverse || B != 1)) {
     set_error("launch_line_fft: a real input is for one forward z pass");
     return JRX_ERR_INVALID;
@@ -137,7 +146,12 @@ int launch_line_fft(const double2* in, double2* out, int64_t B, int n0, int n1,
 int fft3d(const double2* in, double2* out, int64_t B, int n0, int n1, int n2,
           bool inverse, double scale, const FftLen& Lx, const FftLen& Ly,
           const FftLen& Lz, hipStream_t s) {
-  int rc = launch_line_fft(in, out, B, n0, n1, n2, 2, inverse, 1.0, Lz, s);
+  int rc;
+  if (n1 == n2 && box_plane_size(n1)) {  // both inner axes in one pass
+    if ((rc = box_planes(in, out, B * n0, inverse, 1.0, Lz, s))) return rc;
+    return launch_line_fft(out, out, B, n0, n1, n2, 0, inverse, scale, Lx, s);
+  }
+  rc = launch_line_fft(in, out, B, n0, n1, n2, 2, inverse, 1.0, Lz, s);
   if (rc) return rc;
   rc = launch_line_fft(out, out, B, n0, n1, n2, 1, inverse, 1.0, Ly, s);
   if (rc) return rc;
@@ -147,8 +161,14 @@ int fft3d(const double2* in, double2* out, int64_t B, int n0, int n1, int n2,
 int fft3d_real_forward(const double* rin, int ns, double2* out, int n0,
                        int n1, int n2, const FftLen& Lx, const FftLen& Ly,
                        const FftLen& Lz, hipStream_t s) {
-  int rc = launch_line_fft(nullptr, out, 1, n0, n1, n2, 2, false, 1.0, Lz, s,
-                           rin, ns);
+  int rc;
+  if (n1 == n2 && box_plane_size(n1)) {
+    if ((rc = box_planes(nullptr, out, n0, false, 1.0, Lz, s, rin, ns)))
+      return rc;
+    return launch_line_fft(out, out, 1, n0, n1, n2, 0, false, 1.0, Lx, s);
+  }
+  rc = launch_line_fft(nullptr, out, 1, n0, n1, n2, 2, false, 1.0, Lz, s, rin,
+                       ns);
   if (rc) return rc;
   rc = launch_line_fft(out, out, 1, n0, n1, n2, 1, false, 1.0, Ly, s);
   if (rc) return rc;

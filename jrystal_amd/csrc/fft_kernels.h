@@ -53,6 +53,18 @@ int fft3d_real_forward(const double* rin, int ns, double2* out, int n0,
                        int n1, int n2, const FftLen& Lx, const FftLen& Ly,
                        const FftLen& Lz, hipStream_t s);
 
+// Full-box transforms by register lines (boxfft.hip): sizes covered by one-axis
+// passes and by (n x n) planes, and their launchers (L.n is the length; lines
+// as in BoxLine::run).
+bool box_line_size(int n);
+bool box_plane_size(int n);
+int box_line(const double2* in, double2* out, int64_t nouter, int64_t os,
+             int64_t Q, int64_t qs, int64_t es, bool inverse, double scale,
+             const FftLen& L, hipStream_t s);
+int box_planes(const double2* in, double2* out, int64_t B, bool inverse,
+               double scale, const FftLen& L, hipStream_t s,
+               const double* rin = nullptr, int ns = 0);
+
 // T[c][xi][y][z] = 2D inverse transform over (y,z) of the scattered plane
 // x = plane_x[xi] of state (state0 + c); q is band-major [state][ng].
 int launch_plane_ifft(const double2* q, double2* T, int64_t state0,

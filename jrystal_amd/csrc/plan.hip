@@ -1128,6 +1128,12 @@ static int potential_stage(jrx_plan* p, double* rho, double* v, char* ws,
   const FftLen& L0 = p->rowpath ? p->Lz : p->Lx;
   const FftLen& L1 = p->rowpath ? p->Lx : p->Ly;
   const FftLen& L2 = p->rowpath ? p->Ly : p->Lz;
+  if (p->xc == JRX_XC_LDA_X && box_potential_size(cpb)) {
+    JRX_T(JRX_K_POTENTIAL,
+          box_potential_lda(rho, box, v, eh, ee, exc, p->ns, p->cx, ks, cpb,
+                            p->d_sterm, L0, L1, nrec, nexc, s));
+    return JRX_OK;
+  }
   JRX_T(JRX_K_POTENTIAL, fft3d_real_forward(rho, p->ns, box, cpb.nx, cpb.ny,
                                             cpb.nz, L0, L1, L2, s));
   double2* gb = p->o_gb ? cptr(p->o_gb) : nullptr;

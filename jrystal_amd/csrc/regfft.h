@@ -1,7 +1,6 @@
 // Register transforms of one line of N points on L lanes of a wavefront.
 //
-// N = V * L.  Lane j of a line holds x[j + L m] in v[m] (m < V).  The inverse
-// transform runs a V-point DFT over m in registers, multiplies by w_N^{ja},
+// N = V * L.  Lane j of a line holds x[j + L m] in v[m] (m < V).  to_ab runs a V-point DFT over m in registers, multiplies by w_N^{ja},
 // transposes blocks of L registers over the L lanes, and runs W = ceil(V / L)
 // L-point DFTs: lane i ends with X[a + V b] in v[u L + b], a = i + L u
 // (u < W; where a >= V the lane holds nothing of use).  The forward transform
@@ -376,11 +375,13 @@ struct RegLine {
 
   // v <- the line transformed (natural order in, X[a + V b] in v[u L + b]
   // out); x: the line's exchange slots (unused in registers).
-  __device__ __forceinline__ static void inverse(double2 (&v)[VP], double* x,
-                                                 int j, const Tw& tw) {
-    RDft<V, true>::run(v);
+  template <bool INV>
+  __device__ __forceinline__ static void to_ab(double2 (&v)[VP], double* x,
+                                               int j, const Tw& tw) {
+    RDft<V, INV>::run(v);
 #pragma unroll
-    for (int a = 1; a < V; ++a) v[a] = cmulc(tw.w[a], v[a]);
+    for (int a = 1; a < V; ++a)
+      v[a] = INV ? cmulc(tw.w[a], v[a]) : cmul(tw.w[a], v[a]);
     if constexpr (kReg) {
 #pragma unroll
       for (int a = V; a < VP; ++a) v[a] = czero();
@@ -409,15 +410,16 @@ struct RegLine {
       wave_sync();
     }
 #pragma unroll
-    for (int u = 0; u < W; ++u) RDft<L, true>::run(v + u * L);
+    for (int u = 0; u < W; ++u) RDft<L, INV>::run(v + u * L);
   }
 
-  // The forward mirror image: X[a + V b] in v[u L + b] in, natural order out
+  // The mirror image: X[a + V b] in v[u L + b] in, natural order out
   // (v[0 .. V-1]).
-  __device__ __forceinline__ static void forward(double2 (&v)[VP], double* x,
+  template <bool INV>
+  __device__ __forceinline__ static void from_ab(double2 (&v)[VP], double* x,
                                                  int j, const Tw& tw) {
 #pragma unroll
-    for (int u = 0; u < W; ++u) RDft<L, false>::run(v + u * L);
+    for (int u = 0; u < W; ++u) RDft<L, INV>::run(v + u * L);
     if constexpr (kReg) {
       transpose_regs(v);
     } else {
@@ -445,8 +447,35 @@ struct RegLine {
       wave_sync();
     }
 #pragma unroll
-    for (int a = 1; a < V; ++a) v[a] = cmul(tw.w[a], v[a]);
-    RDft<V, false>::run(v);
+    for (int a = 1; a < V; ++a)
+      v[a] = INV ? cmulc(tw.w[a], v[a]) : cmul(tw.w[a], v[a]);
+    RDft<V, INV>::run(v);
+  }
+  __device__ __forceinline__ static void inverse(double2 (&v)[VP], double* x,
+                                                 int j, const Tw& tw) {
+    to_ab<true>(v, x, j, tw);
+  }
+  __device__ __forceinline__ static void forward(double2 (&v)[VP], double* x,
+                                                 int j, const Tw& tw) {
+    from_ab<false>(v, x, j, tw);
+  }
+};
+
+// Lane of a wave -> (line of the block, lane of the line).
+template <int N>
+struct LaneMap {
+  int j, l, wave;
+  bool on;
+  __device__ __forceinline__ LaneMap() {
+    using F = RegLine<N>;
+    const int lane = threadIdx.x & 63;
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    on = F::kLanes == 64 || lane < F::kLanes;
+    l = F::line_of(lane);
+    j = on ? F::j_of(lane) : 0;
+  }
+  __device__ __forceinline__ int line() const {
+    return wave * RegLine<N>::LPW + l;
   }
 };
 

@@ -101,24 +101,6 @@ struct Window {
   static constexpr int WS = (M * L) | 1;  // LDS stride of a row's window
 };
 
-// Lane of a wave -> (line of the block, lane of the line).
-template <int N>
-struct LaneMap {
-  int j, l, wave;
-  bool on;
-  __device__ __forceinline__ LaneMap() {
-    using F = RegLine<N>;
-    const int lane = threadIdx.x & 63;
-    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    on = F::kLanes == 64 || lane < F::kLanes;
-    l = F::line_of(lane);
-    j = on ? F::j_of(lane) : 0;
-  }
-  __device__ __forceinline__ int line() const {
-    return wave * RegLine<N>::LPW + l;
-  }
-};
-
 // ---------------------------------------------------------- row passes --
 // LDS of a row pass: the windows of the block's rows, or (sizes that
 // exchange through LDS) the rows' exchange slots, whichever is larger; the

@@ -714,7 +714,6 @@ int jrx_qr(const double* w_re, const double* w_im, int64_t P, int ng, int nb,
   double2* part = (double2*)(ws + op);
   double2* S = (double2*)(ws + os);
   double2* R1 = (double2*)(ws + oa);
-  double2* R2 = (double2*)(ws + ob);
   const GramSplit sp = gram_split(P, ng, nb);
   hipStream_t s = (hipStream_t)stream;
   int rc;
@@ -724,8 +723,8 @@ int jrx_qr(const double* w_re, const double* w_im, int64_t P, int ng, int nb,
       (rc = launch_gram_gmajor(w_re, w_im, R1, part, P, ng, nb, sp, s, nullptr,
                                (double2*)q)) ||
       (rc = launch_reduce_partials(part, S, P, sp.nchunk, nb, s)) ||
-      (rc = launch_chol_inv(S, R2, P, nb, s)) ||
-      (rc = launch_trmm_uu(R1, R2, (double2*)rinv, P, nb, s)) ||
+      (rc = launch_chol_inv(S, (double2*)rinv, P, nb, s, nullptr, nullptr,
+                            R1)) ||
       (rc = launch_apply_fwd(w_re, w_im, (const double2*)rinv, (double2*)q, P,
                              ng, nb, s)))
     return rc;

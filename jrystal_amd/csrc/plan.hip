@@ -147,7 +147,7 @@ struct jrx_plan {
   size_t o_gb = 0;  // density-gradient boxes of GGA terms [3][N] complex
   size_t o_ritz = 0;  // scratch of the Rayleigh-Ritz rotation
   size_t o_stats;
-  size_t o_q, o_qbar, o_T, o_rho, o_rpart, o_v, o_box, o_tb, o_S, o_R1, o_R2, o_Ri, o_A,
+  size_t o_q, o_qbar, o_T, o_rho, o_rpart, o_v, o_box, o_tb, o_S, o_R1, o_Ri, o_A,
       o_Bm, o_part, o_kin, o_eh, o_ee, o_exc, o_qrflag, o_bepart, o_pot,
       total;
 };
@@ -443,7 +443,6 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->o_box = take((size_t)p->N * sizeof(double2));
   p->o_S = take(mat);
   p->o_R1 = take(mat);
-  p->o_R2 = take(mat);
   p->o_Ri = take(mat);
   p->o_A = take(mat);
   p->o_Bm = take(mat);
@@ -1204,7 +1203,6 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
   double* v = dptr(p->o_v);
   double2* Sm = cptr(p->o_S);
   double2* R1 = cptr(p->o_R1);
-  double2* R2 = cptr(p->o_R2);
   double2* Ri = cptr(p->o_Ri);
   double2* Am = cptr(p->o_A);
   double2* Bm = cptr(p->o_Bm);
@@ -1231,13 +1229,9 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
   JRX_T(JRX_K_QR_SMALL, launch_reduce_partials(part, Sm, P, p->gsw.nchunk, nb, s));
   JRX_T(JRX_K_QR_SMALL, launch_chol_inv(Sm, R1, P, nb, s, one_pass));
   JRX_T(JRX_K_QR_GRAM, launch_gram_gmajor(w_re, w_im, R1, part, P, ng, nb, p->gsw, s, one_pass, q));
-  JRX_T(JRX_K_QR_SMALL, launch_reduce_partials(part, Sm, P, p->gsw.nchunk, nb, s));
-  if (nb <= 32) {  // Ri = R1^{-1} R2^{-1} formed by the factorisation
-    JRX_T(JRX_K_QR_SMALL, launch_chol_inv(Sm, Ri, P, nb, s, nullptr, one_pass, R1));
-  } else {
-    JRX_T(JRX_K_QR_SMALL, launch_chol_inv(Sm, R2, P, nb, s, nullptr, one_pass));
-    JRX_T(JRX_K_QR_SMALL, launch_trmm_uu(R1, R2, Ri, P, nb, s));
-  }
+  JRX_T(JRX_K_QR_SMALL, launch_reduce_partials(part, Sm, P, p->gsw.nchunk, nb, s, one_pass));
+  // Ri = R1^{-1} R2^{-1} formed by the factorisation
+  JRX_T(JRX_K_QR_SMALL, launch_chol_inv(Sm, Ri, P, nb, s, nullptr, one_pass, R1));
   JRX_T(JRX_K_QR_APPLY, launch_apply_fwd(w_re, w_im, Ri, q, P, ng, nb, s));
   // --- density -------------------------------------------------------------
   const int64_t SS = (int64_t)p->nk * nb;  // states per spin

@@ -12,6 +12,7 @@
 //   Wbar = (Qbar + Q copyltu(X)) R^-H,  X = triu(-Q^H Qbar),
 //   copyltu(X) = X + X^H - Re diag(X).
 #include "qr_kernels.h"
+#include "qr_mfma.h"
 
 #include <algorithm>
 
@@ -32,17 +33,6 @@ GramSplit gram_split(int64_t P, int ng, int nb) {
   return sp;
 }
 
-
-// ------------------------------------------------------------- FP64 MFMA --
-// v_mfma_f64_16x16x4f64 on one wave: D(16x16) += A(16x4) B(4x16), lane l
-// supplies A[l%16][l/16] and B[l/16][l%16]; accumulator register r of lane
-// l holds D[4r + l/16][l%16].  Complex products are four real products.
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ d4 mfma4(double a, double b, d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ d4 d4zero() { return d4{0.0, 0.0, 0.0, 0.0}; }
 
 // Small nb x nb matrix into LDS, zero-padded to NBP x NBP.
 __device__ __forceinline__ void load_small(double2* dst, const double2* src,
@@ -252,173 +242,6 @@ int launch_gram_wide(const double* wr, const double* wi, const double2* qa,
 #undef JRX_GRAM_WIDE
   JRX_LAUNCH_CHECK();
   return JRX_OK;
-}
-
-constexpr int kCholWideBlock = 1024;
-constexpr int kInvLanes = 8;  // threads per row in the inverse
-
-// Element (i, j), i <= j, of an upper triangle packed row by row.
-__device__ inline int up_index(int i, int j, int nb) {
-  return i * nb - (i * (i - 1)) / 2 + (j - i);
-}
-
-// chol_inv_kernel for nb > 64: the upper triangle, packed, is the only
-// matrix in LDS (132 KB at nb = 128), factored and inverted in place with
-// one barrier per step.
-// Factorisation, step j (right-looking, on the unscaled row j):
-//   A[r][c] -= conj(A[j][r]) A[j][c] / A[j][j]   (j < r <= c),
-// waves over rows r, lanes over columns c; row j itself is scaled to
-// R[j][c] = A[j][c] / sqrt(A[j][j]) during step j + 1, which does not read
-// it (the pivots are kept aside in piv).
-// Inverse, column j (rows are independent given R):
-//   X[j][j] = 1 / R[j][j],  X[i][j] = -sum_{k=i}^{j-1} X[i][k] R[k][j] / R[j][j],
-// kInvLanes threads per row i sharing the sum; column j of R is copied
-// aside (double-buffered) one step ahead, before X overwrites it.
-__global__ __launch_bounds__(kCholWideBlock) void chol_inv_wide_kernel(
-    const double2* __restrict__ S, double2* __restrict__ rinv, int nb,
-    int* __restrict__ flag_out, const int* __restrict__ flag_in) {
-  extern __shared__ double2 sm[];
-  const int np = nb * (nb + 1) / 2;
-  double2* A = sm;
-  double2* col = sm + np;  // [2][nb]
-  double* piv = reinterpret_cast<double*>(col + 2 * nb);  // [nb]
-  double* red = piv + nb;                                  // [B / 64]
-  const int64_t p = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int B = kCholWideBlock, NW = B / 64;
-  double2* out = rinv + p * nb * nb;
-  if (flag_in && flag_in[p]) {  // uniform over the block
-    for (int e = tid; e < nb * nb; e += B) {
-      const int i = e / nb, j = e - i * nb;
-      out[e] = make_double2(i == j ? 1.0 : 0.0, 0.0);
-    }
-    return;
-  }
-  const double2* Sp = S + p * nb * nb;
-  for (int e = tid; e < nb * nb; e += B) {
-    const int i = e / nb, j = e - i * nb;
-    if (j >= i) A[up_index(i, j, nb)] = Sp[e];
-  }
-  __syncthreads();
-  if (flag_out) {  // distance of the scaled Gram matrix from I
-    double a = 0.0;
-    for (int e = tid; e < nb * nb; e += B) {
-      const int i = e / nb, j = e - i * nb;
-      if (i < j) {  // (i, j) and (j, i)
-        const double2 v = A[up_index(i, j, nb)];
-        a += 2.0 * (v.x * v.x + v.y * v.y) /
-             (A[up_index(i, i, nb)].x * A[up_index(j, j, nb)].x);
-      }
-    }
-    const double d2 = block_sum(a, red);
-    if (tid == 0) flag_out[p] = (d2 < kQrOnePass * kQrOnePass) ? 1 : 0;
-  }
-  // NaN for a non-positive pivot: sqrt of a negative number.
-  auto root = [](double d) { return d > 0.0 ? sqrt(d) : sqrt(-1.0 - d * 0.0); };
-  for (int j = 0; j <= nb; ++j) {
-    if (j >= 1) {  // scale row j - 1 (its pivot is piv[j - 1])
-      const int jm = j - 1, base = up_index(jm, jm, nb);
-      const double sq = root(piv[jm]);
-      for (int c = tid; c < nb - jm; c += B)
-        A[base + c] = c == 0 ? make_double2(sq, 0.0) : cscale(A[base + c], 1.0 / sq);
-    }
-    if (j < nb) {
-      const int base = up_index(j, j, nb);
-      const double dd = A[base].x;
-      if (tid == 0) piv[j] = dd;
-      const double inv = 1.0 / dd;
-      // two rows per pass, every load issued before the stores (nb <= 128:
-      // columns r + lane and r + lane + 64 cover a row)
-      for (int r = j + 1 + wave; r < nb; r += 2 * NW) {
-        const int r2 = r + NW;
-        const bool two = r2 < nb;
-        double2 x[2][2], y[2][2], f[2];
-        int rb[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int rr = h ? (two ? r2 : r) : r;
-          const double2 ajr = A[base + rr - j];
-          f[h] = make_double2(ajr.x * inv, -ajr.y * inv);  // conj / dd
-          rb[h] = up_index(rr, rr, nb);
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int c = rr + lane + 64 * u;
-            x[h][u] = c < nb ? A[rb[h] + c - rr] : czero();
-            y[h][u] = c < nb ? A[base + c - j] : czero();
-          }
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (h && !two) break;
-          const int rr = h ? r2 : r;
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int c = rr + lane + 64 * u;
-            if (c < nb) A[rb[h] + c - rr] = csub(x[h][u], cmul(f[h], y[h][u]));
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // inverse, in place
-  const int i = tid / kInvLanes, t = tid % kInvLanes;
-  const int ib = i < nb ? up_index(i, i, nb) : 0;
-  if (tid <= 0) col[0] = A[0];  // column 0 of R
-  __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    const double2* cj = col + (j & 1) * nb;
-    if (i < j) {
-      double2 acc = czero(), acc2 = czero();
-      int k = i + t;
-      for (; k + kInvLanes < j; k += 2 * kInvLanes) {
-        acc = cadd(acc, cmul(A[ib + k - i], cj[k]));
-        acc2 = cadd(acc2, cmul(A[ib + k + kInvLanes - i], cj[k + kInvLanes]));
-      }
-      if (k < j) acc = cadd(acc, cmul(A[ib + k - i], cj[k]));
-      acc = cadd(acc, acc2);
-#pragma unroll
-      for (int m = kInvLanes / 2; m > 0; m >>= 1) {
-        acc.x += __shfl_xor(acc.x, m, kInvLanes);
-        acc.y += __shfl_xor(acc.y, m, kInvLanes);
-      }
-      if (t == 0) A[ib + j - i] = cscale(acc, -1.0 / cj[j].x);
-    } else if (i == j && t == 0) {
-      A[ib] = make_double2(1.0 / cj[j].x, 0.0);
-    }
-    if (j + 1 < nb) {  // column j + 1 of R, untouched until the next step
-      double2* cn = col + ((j + 1) & 1) * nb;
-      for (int k = tid; k <= j + 1; k += B) cn[k] = A[up_index(k, j + 1, nb)];
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < nb * nb; e += B) {
-    const int r = e / nb, c = e - r * nb;
-    out[e] = (c >= r) ? A[up_index(r, c, nb)] : czero();
-  }
-}
-
-// qr_bwd_small_kernel for nb > 64: one output entry per thread, operands
-// read from global memory (L2-resident nb x nb matrices).
-__global__ __launch_bounds__(kQrBlock) void qr_bwd_small_wide_kernel(
-    const double2* __restrict__ G, const double2* __restrict__ rinv,
-    double2* __restrict__ A, double2* __restrict__ Bm, int nb) {
-  const int64_t p = blockIdx.y;
-  const int e = blockIdx.x * kQrBlock + threadIdx.x;
-  if (e >= nb * nb) return;
-  const int i = e / nb, j = e - i * nb;
-  const double2* Gp = G + p * nb * nb;
-  const double2* Rp = rinv + p * nb * nb;
-  A[p * nb * nb + e] = cconj(Rp[j * nb + i]);
-  double2 acc = czero();
-  for (int k = j; k < nb; ++k) {
-    double2 m;  // copyltu(triu(-G))[i][k]
-    if (i < k) m = make_double2(-Gp[i * nb + k].x, -Gp[i * nb + k].y);
-    else if (i > k) m = make_double2(-Gp[k * nb + i].x, Gp[k * nb + i].y);
-    else m = make_double2(-Gp[i * nb + i].x, 0.0);
-    acc = cadd(acc, cmul(m, cconj(Rp[j * nb + k])));
-  }
-  Bm[p * nb * nb + e] = acc;
 }
 
 constexpr int kWideRows = 64;  // g rows per block of the wide apply kernels
@@ -833,9 +656,10 @@ constexpr int kRedOut = 32, kRedGroups = kQrBlock / kRedOut;
 
 __global__ __launch_bounds__(kQrBlock) void reduce_partials_kernel(
     const double2* __restrict__ partial, double2* __restrict__ out,
-    int nchunk, int nout) {
+    int nchunk, int nout, const int* __restrict__ skip) {
   __shared__ double2 acc[kRedGroups][kRedOut];
   const int64_t p = blockIdx.y;
+  if (skip && skip[p]) return;  // uniform over the block
   const int ol = threadIdx.x % kRedOut, grp = threadIdx.x / kRedOut;
   const int o = blockIdx.x * kRedOut + ol;
   // four independent sums in flight, added in a fixed order
@@ -861,351 +685,15 @@ __global__ __launch_bounds__(kQrBlock) void reduce_partials_kernel(
 }
 
 int launch_reduce_partials(const double2* partial, double2* out, int64_t P,
-                           int nchunk, int nb, hipStream_t s) {
+                           int nchunk, int nb, hipStream_t s,
+                           const int* skip) {
   const int nout = nb * nb;
   dim3 grid(ceil_div(nout, kRedOut), (unsigned)P), block(kQrBlock);
   hipLaunchKernelGGL(reduce_partials_kernel, grid, block, 0, s, partial, out,
-                     nchunk, nout);
+                     nchunk, nout, skip);
   JRX_LAUNCH_CHECK();
   return JRX_OK;
 }
-
-// One block per problem: the Cholesky factor of S = R^H R (R upper) and
-// rinv = X = R^{-1}, in one sweep of nb + 3 steps with one barrier each.
-// Step s:
-//  (a) updates the trailing rows with the unscaled pivot row s,
-//      A[r][c] -= conj(A[s][r]) A[s][c] / A[s][s];
-//  (b) scales row s - 1 into R (R[j][j] = sqrt of the pivot, NaN for a
-//      non-positive one);
-//  (c) adds row x = s - 2 of R into the partial sums of X R = I: with
-//      X[i][c] holding P[i][c] = sum_{k<x} X[i][k] R[k][c] for c >= x,
-//      X[i][c] += X_ix R[x][c] (c > x), X_ix = -P[i][x] / R[x][x]
-//      (1 / R[x][x] for i = x);
-//  (d) writes column y = s - 3 of X from its complete partial sums.
-// (a) writes rows > s of A, (b) row s - 1, (c) and (d) read rows <= s - 2;
-// (c) writes columns > s - 2 of X and (d) column s - 3, so the parts of a
-// step touch disjoint data.  A (then R) and X live in LDS ([nb][nb+1]
-// each).
-__global__ __launch_bounds__(kQrBlock) void chol_inv_kernel(
-    const double2* __restrict__ S, double2* __restrict__ rinv, int nb,
-    int* __restrict__ flag_out, const int* __restrict__ flag_in) {
-  extern __shared__ double2 sm[];
-  __shared__ double dg[kNarrowBands];  // R[j][j]
-  const int ld = nb + 1;
-  double2* A = sm;
-  double2* X = sm + nb * ld;
-  const int64_t p = blockIdx.x;
-  const int tid = threadIdx.x;
-  double2* out = rinv + p * nb * nb;
-  if (flag_in && flag_in[p]) {  // uniform over the block
-    for (int e = tid; e < nb * nb; e += kQrBlock) {
-      const int i = e / nb, j = e - i * nb;
-      out[e] = make_double2(i == j ? 1.0 : 0.0, 0.0);
-    }
-    return;
-  }
-  const double2* Sp = S + p * nb * nb;
-  for (int e = tid; e < nb * nb; e += kQrBlock) {
-    const int i = e / nb, j = e - i * nb;
-    A[i * ld + j] = Sp[e];
-  }
-  __syncthreads();
-  if (flag_out) {  // distance of the scaled Gram matrix from I
-    double a = 0.0;
-    for (int e = tid; e < nb * nb; e += kQrBlock) {
-      const int i = e / nb, j = e - i * nb;
-      if (i != j) {
-        const double2 v = A[i * ld + j];
-        a += (v.x * v.x + v.y * v.y) / (A[i * ld + i].x * A[j * ld + j].x);
-      }
-    }
-    // X is free until the sweep
-    const double d2 = block_sum(a, reinterpret_cast<double*>(X));
-    if (tid == 0)  // NaN or a non-positive diagonal compares false
-      flag_out[p] = (d2 < kQrOnePass * kQrOnePass) ? 1 : 0;
-  }
-  for (int e = tid; e < nb * nb; e += kQrBlock) {
-    const int i = e / nb, j = e - i * nb;
-    X[i * ld + j] = czero();
-  }
-  __syncthreads();
-  for (int st = 0; st < nb + 3; ++st) {
-    if (st < nb) {  // (a)
-      const double piv = A[st * ld + st].x;
-      const double inv = 1.0 / piv;
-      if (tid == 0)  // NaN for a non-positive pivot: sqrt of a negative number
-        dg[st] = piv > 0.0 ? sqrt(piv) : sqrt(-1.0 - piv * 0.0);
-      const int m = nb - st - 1;
-      for (int e = tid; e < m * m; e += kQrBlock) {
-        const int r = st + 1 + e / m, c = st + 1 + e % m;
-        if (c >= r)
-          A[r * ld + c] = csub(A[r * ld + c],
-                               cscale(cmulc(A[st * ld + r], A[st * ld + c]), inv));
-      }
-    }
-    if (st >= 1 && st <= nb) {  // (b)
-      const int j = st - 1;
-      const double d = dg[j];
-      const double id = 1.0 / d;
-      for (int c = j + tid; c < nb; c += kQrBlock)
-        A[j * ld + c] = c == j ? make_double2(d, 0.0) : cscale(A[j * ld + c], id);
-    }
-    if (st >= 2 && st <= nb + 1) {  // (c)
-      const int x = st - 2, w = nb - x - 1;
-      const double ir = 1.0 / A[x * ld + x].x;
-      for (int e = tid; e < (x + 1) * w; e += kQrBlock) {
-        const int i = e / w, c = x + 1 + e % w;
-        const double2 xi = i == x ? make_double2(ir, 0.0)
-                                  : cscale(X[i * ld + x], -ir);
-        X[i * ld + c] = cadd(X[i * ld + c], cmul(xi, A[x * ld + c]));
-      }
-    }
-    if (st >= 3) {  // (d)
-      const int y = st - 3;
-      const double ir = 1.0 / A[y * ld + y].x;
-      for (int i = tid; i <= y; i += kQrBlock)
-        X[i * ld + y] = i == y ? make_double2(ir, 0.0)
-                               : cscale(X[i * ld + y], -ir);
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < nb * nb; e += kQrBlock) {
-    const int i = e / nb, j = e - i * nb;
-    out[e] = (j >= i) ? X[i * ld + j] : czero();
-  }
-}
-
-// chol_inv_kernel for nb <= 32 with the matrices in registers: thread
-// (ty, tx) = (tid / 16, tid % 16) owns rows {ty, ty + 16} x columns
-// {tx, tx + 16} of A and of X = R^{-1}.  The same sweep as chol_inv_kernel
-// (right-looking Cholesky; X from the partial sums of X R = I), with the
-// data that crosses threads passed through LDS buffers that are each written
-// once, ahead of their use: rowbuf[s] = the unscaled pivot row s (written
-// by its owners when step s - 1 has finished it), colbuf[y] = the final
-// column y of X (written at the end of step y + 1).  Step s reads only
-// buffers written before its barrier, so its loads need no ordering with
-// its stores: one barrier per step, nb + 1 steps.
-// 1 / sqrt(a): the hardware estimate refined by one Newton step for
-// f(y) = 1/y^2 - a, y <- y (3 - a y^2) / 2; NaN for a <= 0 (or NaN), so
-// that a non-positive pivot poisons the factor as the IEEE sqrt does.
-__device__ __forceinline__ double rsqrt_newton(double a) {
-  double y = __builtin_amdgcn_rsq(a);
-  y = y * (1.5 - 0.5 * a * y * y);
-  return a > 0.0 ? y : __builtin_nan("");
-}
-
-// With lmul (upper triangular, [P][nb][nb]) the output is lmul X instead
-// of X (the product of the two CholeskyQR2 inverses, summed over k in
-// ascending order as trmm_uu_kernel does).
-__global__ __launch_bounds__(kQrBlock) void chol_inv32_kernel(
-    const double2* __restrict__ S, double2* __restrict__ rinv, int nb,
-    int* __restrict__ flag_out, const int* __restrict__ flag_in,
-    const double2* __restrict__ lmul) {
-  __shared__ double2 rowbuf[32][33];
-  __shared__ double2 colbuf[32][33];
-  __shared__ double red[kQrBlock / 64];
-  const int64_t p = blockIdx.x;
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  double2* out = rinv + p * nb * nb;
-  const double2* L = lmul ? lmul + p * nb * nb : nullptr;
-  if (flag_in && flag_in[p]) {  // uniform over the block: X = I
-    for (int e = tid; e < nb * nb; e += kQrBlock) {
-      const int i = e / nb, j = e - i * nb;
-      out[e] = L ? L[e] : make_double2(i == j ? 1.0 : 0.0, 0.0);
-    }
-    return;
-  }
-  const double2* Sp = S + p * nb * nb;
-  double2 A[4], X[4];
-  int rr[2], cc[2];
-  rr[0] = ty; rr[1] = ty + 16;
-  cc[0] = tx; cc[1] = tx + 16;
-  double dist = 0.0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = rr[q >> 1], c = cc[q & 1];
-    const bool ok = r < nb && c < nb;
-    A[q] = ok ? Sp[r * nb + c] : czero();
-    X[q] = czero();
-    if (ok && r != c)  // distance of the scaled Gram matrix from I
-      dist += (A[q].x * A[q].x + A[q].y * A[q].y) /
-              (Sp[r * nb + r].x * Sp[c * nb + c].x);
-    if (ok && r == 0) rowbuf[0][c] = A[q];
-  }
-  if (flag_out) {
-    const double d2 = block_sum(dist, red);
-    if (tid == 0)  // NaN or a non-positive diagonal compares false
-      flag_out[p] = (d2 < kQrOnePass * kQrOnePass) ? 1 : 0;
-  }
-  __syncthreads();
-  for (int st = 0; st <= nb; ++st) {
-    // Loads, all unconditional (indices clamped into the buffers) so that
-    // they issue back to back; values outside the step's ranges are
-    // selected away below.  Only buffers written before the last barrier
-    // are read.
-    const int sa = st < nb ? st : nb - 1;
-    const int x = st - 2, xa = x < 0 ? 0 : (x < nb ? x : nb - 1);
-    const int y = st - 1, ya = y < 0 ? 0 : (y < nb ? y : nb - 1);
-    const double pst = rowbuf[sa][sa].x, px = rowbuf[xa][xa].x,
-                 py = rowbuf[ya][ya].x;
-    double2 sr[2], sc[2], rx[2], xi[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      sr[a] = rowbuf[sa][rr[a]];
-      sc[a] = rowbuf[sa][cc[a]];
-      rx[a] = rowbuf[xa][cc[a]];
-      xi[a] = colbuf[xa][rr[a]];
-    }
-    const double ys = rsqrt_newton(pst);
-    const double inv = ys * ys;                 // 1 / pivot
-    const double idx = rsqrt_newton(px);        // 1 / R[x][x]
-    const double iy = rsqrt_newton(py);         // 1 / R[y][y]
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int a = q >> 1, b = q & 1;
-      const int r = rr[a], c = cc[b];
-      // Cholesky update with pivot row st
-      if (st < nb && r > st && c >= r && c < nb)
-        A[q] = csub(A[q], cscale(cmulc(sr[a], sc[b]), inv));
-      // row x of R into the partial sums of X
-      if (x >= 0 && r <= x && c > x && c < nb)
-        X[q] = cadd(X[q], cmul(xi[a], cscale(rx[b], idx)));
-      // row st + 1 is final: publish it
-      if (st + 1 < nb && r == st + 1 && c >= r && c < nb)
-        rowbuf[st + 1][c] = A[q];
-      // column y of X is complete: finalise and publish it
-      if (y >= 0 && y < nb && c == y && r <= y) {
-        X[q] = r == y ? make_double2(iy, 0.0) : cscale(X[q], -iy);
-        colbuf[y][r] = X[q];
-      }
-    }
-    __syncthreads();
-  }
-  if (L) {  // X into LDS (the loop's last barrier has retired colbuf)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = rr[q >> 1], c = cc[q & 1];
-      colbuf[r][c] = (r < nb && c < nb && c >= r) ? X[q] : czero();
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = rr[q >> 1], c = cc[q & 1];
-      if (r < nb && c < nb) {
-        double2 acc = czero();
-        for (int k = r; k <= c; ++k) acc = cadd(acc, cmul(L[r * nb + k], colbuf[k][c]));
-        out[r * nb + c] = acc;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = rr[q >> 1], c = cc[q & 1];
-    if (r < nb && c < nb) out[r * nb + c] = c >= r ? X[q] : czero();
-  }
-}
-
-int launch_chol_inv(const double2* S, double2* rinv, int64_t P, int nb,
-                    hipStream_t s, int* flag_out, const int* flag_in,
-                    const double2* lmul) {
-  if (lmul && nb > 32) {
-    set_error("launch_chol_inv: lmul is for at most 32 bands");
-    return JRX_ERR_INVALID;
-  }
-  if (nb > kNarrowBands) {
-    const size_t shm = ((size_t)nb * (nb + 1) / 2 + 2 * nb) * sizeof(double2) +
-                       (nb + kCholWideBlock / 64) * sizeof(double);
-    hipLaunchKernelGGL(chol_inv_wide_kernel, dim3((unsigned)P),
-                       dim3(kCholWideBlock), shm, s, S, rinv, nb, flag_out,
-                       flag_in);
-    JRX_LAUNCH_CHECK();
-    return JRX_OK;
-  }
-  if (nb <= 32) {
-    hipLaunchKernelGGL(chol_inv32_kernel, dim3((unsigned)P), dim3(kQrBlock), 0,
-                       s, S, rinv, nb, flag_out, flag_in, lmul);
-    JRX_LAUNCH_CHECK();
-    return JRX_OK;
-  }
-  size_t shm = 2 * (size_t)nb * (nb + 1) * sizeof(double2);
-  hipLaunchKernelGGL(chol_inv_kernel, dim3((unsigned)P), dim3(kQrBlock), shm,
-                     s, S, rinv, nb, flag_out, flag_in);
-  JRX_LAUNCH_CHECK();
-  return JRX_OK;
-}
-
-__global__ __launch_bounds__(kQrBlock) void trmm_uu_kernel(
-    const double2* __restrict__ a, const double2* __restrict__ b,
-    double2* __restrict__ c, int nb) {
-  const int64_t p = blockIdx.y;
-  const int e = blockIdx.x * kQrBlock + threadIdx.x;
-  if (e >= nb * nb) return;
-  const int i = e / nb, j = e - i * nb;
-  const double2* ap = a + p * nb * nb;
-  const double2* bp = b + p * nb * nb;
-  double2 acc = czero();
-  for (int k = i; k <= j; ++k) acc = cadd(acc, cmul(ap[i * nb + k], bp[k * nb + j]));
-  c[p * nb * nb + e] = acc;
-}
-
-int launch_trmm_uu(const double2* a, const double2* b, double2* c, int64_t P,
-                   int nb, hipStream_t s) {
-  dim3 grid(ceil_div(nb * nb, kQrBlock), (unsigned)P), block(kQrBlock);
-  hipLaunchKernelGGL(trmm_uu_kernel, grid, block, 0, s, a, b, c, nb);
-  JRX_LAUNCH_CHECK();
-  return JRX_OK;
-}
-
-__global__ __launch_bounds__(kQrBlock) void qr_bwd_small_kernel(
-    const double2* __restrict__ G, const double2* __restrict__ rinv,
-    double2* __restrict__ A, double2* __restrict__ Bm, int nb) {
-  extern __shared__ double2 sm[];
-  const int ld = nb + 1;
-  double2* M = sm;             // copyltu(triu(-G))
-  double2* Ri = sm + nb * ld;  // R^{-1}
-  const int64_t p = blockIdx.x;
-  const int tid = threadIdx.x;
-  const double2* Gp = G + p * nb * nb;
-  const double2* Rp = rinv + p * nb * nb;
-  for (int e = tid; e < nb * nb; e += kQrBlock) {
-    const int i = e / nb, j = e - i * nb;
-    double2 m;
-    if (i < j) m = make_double2(-Gp[e].x, -Gp[e].y);
-    else if (i > j) m = make_double2(-Gp[j * nb + i].x, Gp[j * nb + i].y);
-    else m = make_double2(-Gp[e].x, 0.0);
-    M[i * ld + j] = m;
-    Ri[i * ld + j] = Rp[e];
-  }
-  __syncthreads();
-  double2* Ap = A + p * nb * nb;
-  double2* Bp = Bm + p * nb * nb;
-  for (int e = tid; e < nb * nb; e += kQrBlock) {
-    const int i = e / nb, j = e - i * nb;
-    // (R^-H)[k][j] = conj(Ri[j][k]), nonzero for k >= j
-    Ap[e] = i >= j ? cconj(Ri[j * ld + i]) : czero();
-    double2 acc = czero();
-    for (int k = j; k < nb; ++k) acc = cadd(acc, cmul(M[i * ld + k], cconj(Ri[j * ld + k])));
-    Bp[e] = acc;
-  }
-}
-
-int launch_qr_bwd_small(const double2* G, const double2* rinv, double2* A,
-                        double2* Bm, int64_t P, int nb, hipStream_t s) {
-  if (nb > kNarrowBands) {
-    hipLaunchKernelGGL(qr_bwd_small_wide_kernel,
-                       dim3(ceil_div(nb * nb, kQrBlock), (unsigned)P),
-                       dim3(kQrBlock), 0, s, G, rinv, A, Bm, nb);
-    JRX_LAUNCH_CHECK();
-    return JRX_OK;
-  }
-  size_t shm = 2 * (size_t)nb * (nb + 1) * sizeof(double2);
-  hipLaunchKernelGGL(qr_bwd_small_kernel, dim3((unsigned)P), dim3(kQrBlock),
-                     shm, s, G, rinv, A, Bm, nb);
-  JRX_LAUNCH_CHECK();
-  return JRX_OK;
-}
-
 
 // Rows per block of the narrow apply kernels: 256, halved (down to 64)
 // while the grid would hold fewer than 2048 blocks, so that problems with
@@ -1458,13 +946,12 @@ __global__ __launch_bounds__(kQrBlock) void apply_bwd_kernel(
 
 size_t qr_lds_bytes(int nb) {
   const size_t nbp = 16 * (size_t)((nb + 15) / 16), z = sizeof(double2);
-  if (nb <= kNarrowBands)  // Gram (pre + sums), apply_bwd, chol_inv
-    return std::max(2 * nbp * nbp * z, 2 * (size_t)nb * (nb + 1) * z);
+  const size_t chol = chol_inv_lds_bytes(nb);
+  if (nb <= kNarrowBands)  // Gram (pre + sums), apply_bwd
+    return std::max(2 * nbp * nbp * z, chol);
   const size_t gram = 2 * 2 * (size_t)wide_slab<false>() * (nbp + 1) * z;
   const size_t fwd = (size_t)kWideK * nbp * z;
   const size_t bwd = 2 * (size_t)kWideKB * nbp * z;
-  const size_t chol = ((size_t)nb * (nb + 1) / 2 + 2 * nb) * z +
-                      (nb + kCholWideBlock / 64) * sizeof(double);
   return std::max(std::max(gram, fwd), std::max(bwd, chol));
 }
 

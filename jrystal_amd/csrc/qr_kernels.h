@@ -44,9 +44,11 @@ int launch_gram_bmajor(const double2* q, const double2* qb, double2* partial,
                        int64_t P, int ng, int nb, const GramSplit& sp,
                        hipStream_t s);
 
-// out[p] = sum_c partial[p][c] (fixed order).
+// out[p] = sum_c partial[p][c] (fixed order); problems with skip[p] != 0
+// are left out.
 int launch_reduce_partials(const double2* partial, double2* out, int64_t P,
-                           int nchunk, int nb, hipStream_t s);
+                           int nchunk, int nb, hipStream_t s,
+                           const int* skip = nullptr);
 
 // S = R^H R (R upper, real positive diagonal); writes R^{-1}.  A
 // non-positive pivot turns the result into NaN.
@@ -56,17 +58,14 @@ int launch_reduce_partials(const double2* partial, double2* out, int64_t P,
 // i.e. ||D S D - I||_F < kQrOnePass with D = diag(S)^-1/2, which bounds
 // cond(D S D) by (1 + x) / (1 - x) = 3 and cond(W D) by sqrt(3); else 0.
 // flag_in (optional): problems with flag_in[p] != 0 get R^{-1} = I.
-// lmul (optional, nb <= 32): rinv = lmul R^{-1} for upper-triangular lmul
-// [P][nb][nb] (trmm_uu fused into the factorisation).
+// lmul (optional): rinv = lmul R^{-1} for upper-triangular lmul [P][nb][nb].
 constexpr double kQrOnePass = 0.5;
 int launch_chol_inv(const double2* S, double2* rinv, int64_t P, int nb,
                     hipStream_t s, int* flag_out = nullptr,
                     const int* flag_in = nullptr,
                     const double2* lmul = nullptr);
 
-// c = a * b for upper-triangular a, b.
-int launch_trmm_uu(const double2* a, const double2* b, double2* c, int64_t P,
-                   int nb, hipStream_t s);
+size_t chol_inv_lds_bytes(int nb);
 
 // Q[p][b][g] = sum_i W[p][g][i] rinv[p][i][b] (rinv upper triangular);
 // problems with skip[p] != 0 are left out.

@@ -149,84 +149,136 @@ int launch_potential_real(const double2* vbox, const double* rho, double* v,
 }
 
 // g_m[3g..3g+2] are the integer frequencies (mx, my, mz) of mask point g.
+// Block (state, slice of rows points).
 __global__ __launch_bounds__(kRedBlock) void kinetic_kernel(
-    const double2* __restrict__ q, const double* __restrict__ occ,
-    const double* __restrict__ kpts, const short* __restrict__ g_m,
-    CellParams cp, int ng, int nk, int nb, int gblocks,
-    double* __restrict__ kin_part) {
-  __shared__ double red[kRedBlock];
+    const double2* __restrict__ q, const double* __restrict__ kpts,
+    const short* __restrict__ g_m, CellParams cp, int ng, int nk, int nb,
+    int gblocks, int slice, double* __restrict__ kin_part) {
+  __shared__ double red[kRedBlock / 64];
   const int64_t st = blockIdx.x / gblocks;
   const int gbk = (int)(blockIdx.x % gblocks);
-  const int g = gbk * kRedBlock + threadIdx.x;
+  const int g0 = gbk * slice, g1 = min(ng, g0 + slice);
+  const int k = (int)((st / nb) % nk);
+  const double kx = kpts[3 * k], ky = kpts[3 * k + 1], kz = kpts[3 * k + 2];
+  const double2* qs = q + st * ng;
   double kin = 0.0;
-  if (g < ng) {
-    const int k = (int)((st / nb) % nk);
+#pragma unroll 4
+  for (int g = g0 + threadIdx.x; g < g1; g += kRedBlock) {
     const int mx = g_m[3 * g], my = g_m[3 * g + 1], mz = g_m[3 * g + 2];
-    const double gx = mx * cp.B[0] + my * cp.B[3] + mz * cp.B[6] + kpts[3 * k];
-    const double gy = mx * cp.B[1] + my * cp.B[4] + mz * cp.B[7] + kpts[3 * k + 1];
-    const double gz = mx * cp.B[2] + my * cp.B[5] + mz * cp.B[8] + kpts[3 * k + 2];
-    const double2 c = q[st * ng + g];
-    kin = (gx * gx + gy * gy + gz * gz) * (c.x * c.x + c.y * c.y);
-    (void)occ;
+    const double gx = mx * cp.B[0] + my * cp.B[3] + mz * cp.B[6] + kx;
+    const double gy = mx * cp.B[1] + my * cp.B[4] + mz * cp.B[7] + ky;
+    const double gz = mx * cp.B[2] + my * cp.B[5] + mz * cp.B[8] + kz;
+    const double2 c = qs[g];
+    kin += (gx * gx + gy * gy + gz * gz) * (c.x * c.x + c.y * c.y);
   }
   const double t = block_sum(kin, red);
   if (threadIdx.x == 0) kin_part[st * gblocks + gbk] = t;
 }
 
-int launch_kinetic(const double2* q, const double* occ, const double* kpts,
-                   const short* g_m, const CellParams& cp, int64_t nstates,
-                   int ng, int nk, int nb, double* kin_part, int* nparts,
-                   hipStream_t s) {
-  const int gb = ceil_div(ng, kRedBlock);
-  if ((int64_t)gb * nstates > 0x7fffffff) {
+int launch_kinetic(const double2* q, const double* kpts, const short* g_m,
+                   const CellParams& cp, int64_t nstates, int ng, int nk,
+                   int nb, double* kin_part, int* nper, hipStream_t s) {
+  // one 256-point slice per block while that leaves fewer than about 4096
+  // blocks, else longer slices (fewer partials; a block's reduction costs
+  // as much as a slice of about 500 points)
+  const int all = ceil_div(ng, kRedBlock);
+  int64_t gb = 4096 / nstates;
+  if (gb < 1) gb = 1;
+  if (gb > all) gb = all;
+  const int slice = ceil_div(ceil_div(ng, gb), kRedBlock) * kRedBlock;
+  gb = ceil_div(ng, slice);
+  if (gb * nstates > 0x7fffffff) {
     set_error("too many states for the kinetic reduction");
     return JRX_ERR_UNSUPPORTED;
   }
   hipLaunchKernelGGL(kinetic_kernel, dim3((unsigned)(gb * nstates)),
-                     dim3(kRedBlock), 0, s, q, occ, kpts, g_m, cp, ng, nk, nb,
-                     gb, kin_part);
+                     dim3(kRedBlock), 0, s, q, kpts, g_m, cp, ng, nk, nb,
+                     (int)gb, slice, kin_part);
   JRX_LAUNCH_CHECK();
-  *nparts = (int)(gb * nstates);
+  *nper = (int)gb;
   return JRX_OK;
 }
 
+// Sum of p[0 .. n) over the block, four sums in flight per thread (a fixed
+// order for every n).
+template <int BLOCK>
 __device__ double strided_sum(const double* p, int n, double* red) {
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += kRedBlock) acc += p[i];
-  return block_sum(acc, red);
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
+  int i = threadIdx.x;
+  for (; i + 3 * BLOCK < n; i += 4 * BLOCK)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] += p[i + u * BLOCK];
+  for (; i < n; i += BLOCK) a[0] += p[i];
+  return block_sum((a[0] + a[1]) + (a[2] + a[3]), red);
+}
+
+// Sum of the nper partials of state st on 16 neighbouring lanes (every lane
+// gets it).
+__device__ __forceinline__ double state_sum16(const double* part, int nper,
+                                              int64_t st, int l) {
+  double a = 0.0;
+  for (int j = l; j < nper; j += 16) a += part[st * nper + j];
+#pragma unroll
+  for (int m = 8; m > 0; m >>= 1) a += __shfl_xor(a, m, 16);
+  return a;
 }
 
 // tb[st] = sum_j part[st * nper + j] (fixed order): |G+k|^2-weighted norm
-// of each state, i.e. twice its kinetic energy.
+// of each state, i.e. twice its kinetic energy; 16 lanes per state.
 __global__ __launch_bounds__(kRedBlock) void state_sums_kernel(
     const double* __restrict__ part, int nper, int64_t S,
     double* __restrict__ tb) {
-  const int64_t st = (int64_t)blockIdx.x * kRedBlock + threadIdx.x;
-  if (st >= S) return;
-  double a = 0.0;
-  for (int j = 0; j < nper; ++j) a += part[st * nper + j];
-  tb[st] = a;
+  const int l = threadIdx.x & 15;
+  const int64_t st =
+      (int64_t)blockIdx.x * (kRedBlock / 16) + (threadIdx.x >> 4);
+  if (st >= S) return;  // uniform over the 16 lanes
+  const double a = state_sum16(part, nper, st, l);
+  if (l == 0) tb[st] = a;
 }
 
 int launch_state_sums(const double* part, int nper, int64_t S, double* tb,
                       hipStream_t s) {
-  hipLaunchKernelGGL(state_sums_kernel, dim3(ceil_div(S, kRedBlock)),
+  hipLaunchKernelGGL(state_sums_kernel, dim3(ceil_div(S, kRedBlock / 16)),
                      dim3(kRedBlock), 0, s, part, nper, S, tb);
   JRX_LAUNCH_CHECK();
   return JRX_OK;
 }
 
-__global__ __launch_bounds__(kRedBlock) void finalize_energies_kernel(
-    const double* tb, const double* occ, int64_t S, const double* eh,
+// Thread's share of sum_st occ[st] x[st]; with part the block first forms
+// x[st] from its nper partials (and stores it).
+template <int BLOCK>
+__device__ double occ_sum(const double* __restrict__ part, int nper,
+                          double* x, const double* __restrict__ occ,
+                          int64_t S) {
+  double a = 0.0;
+  if (part) {
+    const int l = threadIdx.x & 15;
+    for (int64_t st = threadIdx.x >> 4; st < S; st += BLOCK / 16) {
+      const double t = state_sum16(part, nper, st, l);
+      if (l == 0) {
+        x[st] = t;
+        a += occ[st] * t;
+      }
+    }
+  } else {
+    for (int64_t i = threadIdx.x; i < S; i += BLOCK) a += occ[i] * x[i];
+  }
+  return a;
+}
+
+constexpr int kFinBlock = 1024;
+
+__global__ __launch_bounds__(kFinBlock) void finalize_energies_kernel(
+    const double* __restrict__ kin, int nper, double* tb,
+    const double* __restrict__ occ, int64_t S, const double* eh,
     const double* ee, int nrec, const double* exc, int nexc,
     double* energies) {
-  __shared__ double red[kRedBlock];
-  double a = 0.0;
-  for (int64_t i = threadIdx.x; i < S; i += kRedBlock) a += occ[i] * tb[i];
-  const double k = 0.5 * block_sum(a, red);
-  const double h = strided_sum(eh, nrec, red);
-  const double e = strided_sum(ee, nrec, red);
-  const double x = strided_sum(exc, nexc, red);
+  __shared__ double red[kFinBlock / 64];
+  const double k =
+      0.5 * block_sum(occ_sum<kFinBlock>(kin, nper, tb, occ, S), red);
+  const double h = strided_sum<kFinBlock>(eh, nrec, red);
+  const double e = strided_sum<kFinBlock>(ee, nrec, red);
+  const double x = strided_sum<kFinBlock>(exc, nexc, red);
   if (threadIdx.x == 0) {
     energies[0] = k;
     energies[1] = h;
@@ -236,12 +288,46 @@ __global__ __launch_bounds__(kRedBlock) void finalize_energies_kernel(
   }
 }
 
-int launch_finalize_energies(const double* tb, const double* occ, int64_t S,
-                             const double* eh, const double* ee, int nrec,
-                             const double* exc, int nexc, double* energies,
-                             hipStream_t s) {
-  hipLaunchKernelGGL(finalize_energies_kernel, dim3(1), dim3(kRedBlock), 0, s,
-                     tb, occ, S, eh, ee, nrec, exc, nexc, energies);
+bool finalize_sums_states(int64_t S, int nper) {
+  return S <= 256 && nper <= 128;
+}
+
+int launch_finalize_energies(const double* kin, int nper, double* tb,
+                             const double* occ, int64_t S, const double* eh,
+                             const double* ee, int nrec, const double* exc,
+                             int nexc, double* energies, hipStream_t s) {
+  hipLaunchKernelGGL(finalize_energies_kernel, dim3(1), dim3(kFinBlock), 0, s,
+                     kin, nper, tb, occ, S, eh, ee, nrec, exc, nexc, energies);
+  JRX_LAUNCH_CHECK();
+  return JRX_OK;
+}
+
+// energies = {sum f tb / 2, sum f pot / vol, 0, 0, their sum}: the band
+// energies' trace sum f <psi|T + v|psi> of the Kohn-Sham band mode.
+__global__ __launch_bounds__(kFinBlock) void band_trace_kernel(
+    const double* __restrict__ kin, const double* __restrict__ pot_part,
+    int nper, double* tb, double* pot, const double* __restrict__ occ,
+    int64_t S, double inv_vol, double* __restrict__ energies) {
+  __shared__ double red[kFinBlock / 64];
+  const double k =
+      0.5 * block_sum(occ_sum<kFinBlock>(kin, nper, tb, occ, S), red);
+  const double u =
+      inv_vol *
+      block_sum(occ_sum<kFinBlock>(pot_part, nper, pot, occ, S), red);
+  if (threadIdx.x == 0) {
+    energies[0] = k;
+    energies[1] = u;
+    energies[2] = 0.0;
+    energies[3] = 0.0;
+    energies[4] = k + u;
+  }
+}
+
+int launch_band_trace(const double* kin, const double* pot_part, int nper,
+                      double* tb, double* pot, const double* occ, int64_t S,
+                      double vol, double* energies, hipStream_t s) {
+  hipLaunchKernelGGL(band_trace_kernel, dim3(1), dim3(kFinBlock), 0, s, kin,
+                     pot_part, nper, tb, pot, occ, S, 1.0 / vol, energies);
   JRX_LAUNCH_CHECK();
   return JRX_OK;
 }

@@ -44,11 +44,11 @@ int launch_potential_real(const double2* vbox, const double* rho, double* v,
                           double cx, int* nparts, hipStream_t s,
                           bool ks = false);
 
-// Partials of |G+k|^2 |q|^2 per (state, g-block), band-major q.
-int launch_kinetic(const double2* q, const double* occ, const double* kpts,
-                   const short* g_m, const CellParams& cp, int64_t nstates,
-                   int ng, int nk, int nb, double* kin_part, int* nparts,
-                   hipStream_t s);
+// Partials of |G+k|^2 |q|^2, *nper per state (at most ceil(ng / kRedBlock)),
+// band-major q.
+int launch_kinetic(const double2* q, const double* kpts, const short* g_m,
+                   const CellParams& cp, int64_t nstates, int ng, int nk,
+                   int nb, double* kin_part, int* nper, hipStream_t s);
 
 // tb[st] = sum_j part[st * nper + j]: sum_G |G+k|^2 |q|^2 of each state
 // (twice the band kinetic energy).
@@ -56,11 +56,20 @@ int launch_state_sums(const double* part, int nper, int64_t S, double* tb,
                       hipStream_t s);
 
 // energies[0..4] = kinetic (1/2 sum occ tb), hartree, external, xc, total
-// from the partials (fixed summation order).
-int launch_finalize_energies(const double* tb, const double* occ, int64_t S,
-                             const double* eh, const double* ee, int nrec,
-                             const double* exc, int nexc, double* energies,
-                             hipStream_t s);
+// from the partials (fixed summation order).  With kin, tb is first formed
+// from its nper partials per state in the same launch; finalize_sums_states
+// says where that one block is quicker than launch_state_sums (up to 256
+// states of 128 partials, four passes of 64 states).
+bool finalize_sums_states(int64_t S, int nper);
+int launch_finalize_energies(const double* kin, int nper, double* tb,
+                             const double* occ, int64_t S, const double* eh,
+                             const double* ee, int nrec, const double* exc,
+                             int nexc, double* energies, hipStream_t s);
+// energies of the band mode: {1/2 sum occ tb, sum occ pot / vol, 0, 0, sum}
+// (kin and pot_part as kin above, both or neither).
+int launch_band_trace(const double* kin, const double* pot_part, int nper,
+                      double* tb, double* pot, const double* occ, int64_t S,
+                      double vol, double* energies, hipStream_t s);
 
 int launch_fill(double* p, double v, int64_t n, hipStream_t s);
 

@@ -1154,29 +1154,6 @@ static int potential_stage(jrx_plan* p, double* rho, double* v, char* ws,
   return JRX_OK;
 }
 
-// energies = {sum f tb / 2, sum f pot / vol, 0, 0, their sum}: the band
-// energies' trace sum f <psi|T + v|psi> of the Kohn-Sham band mode.
-__global__ __launch_bounds__(256) void band_trace_kernel(
-    const double* __restrict__ tb, const double* __restrict__ pot,
-    const double* __restrict__ occ, int64_t S, double inv_vol,
-    double* __restrict__ energies) {
-  __shared__ double red[4];
-  double a = 0.0, b = 0.0;
-  for (int64_t i = threadIdx.x; i < S; i += 256) {
-    a += occ[i] * tb[i];
-    b += occ[i] * pot[i];
-  }
-  const double k = 0.5 * block_sum(a, red);
-  const double u = inv_vol * block_sum(b, red);
-  if (threadIdx.x == 0) {
-    energies[0] = k;
-    energies[1] = u;
-    energies[2] = 0.0;
-    energies[3] = 0.0;
-    energies[4] = k + u;
-  }
-}
-
 // One evaluation into the given workspace; `timed` allows the per-kernel
 // events of jrx_plan_set_timing (their first use creates HIP events).
 static int energy_grad_impl(jrx_plan* p, const double* w_re,
@@ -1239,7 +1216,9 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
   const int64_t plane_elems =
       p->rowpath ? (int64_t)p->nz * p->geo.rstride
                  : (int64_t)p->geo.nxa * p->geo.ps;
-  int nrec = 0, nexc = 0, nkin = 0;
+  int nrec = 0, nexc = 0;
+  int nper = 0;             // kinetic partials per state
+  bool fused_sums = false;  // summed by the final energy kernel
   if (!fixed) {
     for (int sp = 0; sp < p->ns; ++sp) {
       const int64_t step = p->keep_planes ? SS : p->chunk;
@@ -1344,9 +1323,10 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
         }
       }
     }
-    const int nper = p->rowpath ? p->row_chunks : p->geo.nxa;
-    JRX_T(JRX_K_OTHER, launch_state_sums(kin, nper, S, tb, s));
-    if (pot_e)
+    nper = p->rowpath ? p->row_chunks : p->geo.nxa;
+    fused_sums = finalize_sums_states(S, nper);
+    if (!fused_sums) JRX_T(JRX_K_OTHER, launch_state_sums(kin, nper, S, tb, s));
+    if (pot_e && !(fused_sums && fixed))
       JRX_T(JRX_K_OTHER, launch_state_sums(dptr(p->o_bepart), nper, S,
                                            dptr(p->o_pot), s));
     // --- non-local pseudopotential: energy per band and its qbar term ------
@@ -1363,21 +1343,25 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
       JRX_T(JRX_K_QR_BWD_APPLY, launch_apply_bwd(qbar, q, Am, Bm, dw_re, dw_im, P, ng, nb, s));
     }
   } else {
-    JRX_T(JRX_K_OTHER, launch_kinetic(q, p->d_occ, p->d_kpts, p->d_g_m, p->cp, S, ng,
-                           p->nk, nb, kin, &nkin, s));
-    JRX_T(JRX_K_OTHER, launch_state_sums(kin, (int)(nkin / S), S, tb, s));
+    JRX_T(JRX_K_OTHER, launch_kinetic(q, p->d_kpts, p->d_g_m, p->cp, S, ng,
+                                      p->nk, nb, kin, &nper, s));
+    fused_sums = finalize_sums_states(S, nper);
+    if (!fused_sums) JRX_T(JRX_K_OTHER, launch_state_sums(kin, nper, S, tb, s));
     if (p->nproj > 0)
       JRX_T(JRX_K_OTHER, launch_nonlocal(p->d_proj, q, p->d_occ, P, p->nk,
                                          p->nproj, ng, nb, p->vol, nullptr,
                                          p->d_nlscratch, p->d_enl, s));
   }
+  const double* sums = fused_sums ? kin : nullptr;
   if (fixed) {
-    hipLaunchKernelGGL(band_trace_kernel, dim3(1), dim3(256), 0, s, tb,
-                       dptr(p->o_pot), p->d_occ, S, 1.0 / p->vol, energies);
-    JRX_LAUNCH_CHECK();
+    JRX_T(JRX_K_OTHER,
+          launch_band_trace(sums, fused_sums ? dptr(p->o_bepart) : nullptr,
+                            nper, tb, dptr(p->o_pot), p->d_occ, S, p->vol,
+                            energies, s));
   } else {
-    JRX_T(JRX_K_OTHER, launch_finalize_energies(tb, p->d_occ, S, eh, ee, nrec,
-                                                exc, nexc, energies, s));
+    JRX_T(JRX_K_OTHER,
+          launch_finalize_energies(sums, nper, tb, p->d_occ, S, eh, ee, nrec,
+                                   exc, nexc, energies, s));
   }
   if (p->nproj > 0)  // the non-local energy joins the external term
     JRX_T(JRX_K_OTHER, launch_nonlocal_finalize(p->d_enl, p->d_occ, S,

@@ -143,8 +143,9 @@ bool use_rowpath(const BoxGeom& geo);
 // Row blocks of the row passes (the gather writes that many kinetic and
 // band-energy partials per state).
 int row_chunks(const BoxGeom& geo);
-// State groups of a z-plane pass.
-int zplane_groups(const BoxGeom& geo, int nstates);
+// State groups of the z-plane passes (>= 1; not monotonic in nstates).
+int zplane_density_groups(const BoxGeom& geo, int nstates);
+int zplane_vpsi_groups(const BoxGeom& geo, int nstates);
 int launch_row_ifft(const double2* q, double2* R, int64_t state0, int nstates,
                     const BoxGeom& geo, const double2* tw, hipStream_t s);
 // rho_part[g][z][x][y] += sum_{c in group g} occ |psi_c|^2 / vol, or =

@@ -398,7 +398,7 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->qr_adaptive = d->qr_passes == 0;
   p->xline_blocks = d->xline_blocks > 0 ? d->xline_blocks : 0;
   const int sweep_states = p->keep_planes ? (int)spin_states : p->chunk;
-  p->groups = p->rowpath ? zplane_groups(p->geo, sweep_states)
+  p->groups = p->rowpath ? zplane_density_groups(p->geo, sweep_states)
                          : xline_groups(p->geo, sweep_states, p->xline_blocks);
   p->row_chunks = p->rowpath ? row_chunks(p->geo) : 0;
   // z-major cell of the row path: box axes (z, x, y)
@@ -1226,7 +1226,7 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
       // p->groups groups; otherwise the partials start from zero
       const int first = (int)(SS < step ? SS : step);
       const bool store_first =
-          (p->rowpath ? zplane_groups(p->geo, first)
+          (p->rowpath ? zplane_density_groups(p->geo, first)
                       : xline_groups(p->geo, first, p->xline_blocks)) ==
           p->groups;
       if (!store_first)
@@ -1238,10 +1238,12 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
         if (p->rowpath) {
           JRX_T(JRX_K_PLANE_IFFT,
                 launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lz.tw, s));
+          // (a shorter last chunk may ask for more groups than rpart holds)
+          int groups = zplane_density_groups(p->geo, nst);
+          if (groups > p->groups) groups = p->groups;
           JRX_T(JRX_K_XLINE_DENSITY,
-                launch_zplane_density(Tc, rpart, zplane_groups(p->geo, nst),
-                                      p->d_occ, st0, nst, 1.0 / p->vol,
-                                      p->geo, p->Lx.tw,
+                launch_zplane_density(Tc, rpart, groups, p->d_occ, st0, nst,
+                                      1.0 / p->vol, p->geo, p->Lx.tw,
                                       store_first && s0 == 0, s));
         } else if (reg64) {
           JRX_T(JRX_K_PLANE_IFFT, launch_plane_ifft64(q, Tc, st0, nst, p->geo,
@@ -1294,7 +1296,7 @@ static int energy_grad_impl(jrx_plan* p, const double* w_re,
                   launch_row_ifft(q, Tc, st0, nst, p->geo, p->Lz.tw, s));
           JRX_T(JRX_K_XLINE_VPSI,
                 launch_zplane_vpsi(Tc, vv + sp * p->N,
-                                   zplane_groups(p->geo, nst), nst, p->geo,
+                                   zplane_vpsi_groups(p->geo, nst), nst, p->geo,
                                    p->Lx.tw, s));
           JRX_T(JRX_K_PLANE_FFT_GATHER,
                 launch_row_fft_gather(Tc, q, qbar, kin, st0, nst, p->geo,

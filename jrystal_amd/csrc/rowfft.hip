@@ -112,17 +112,63 @@ int row_chunks(const BoxGeom& geo) {
   return (geo.nrows + rpb - 1) / rpb;
 }
 
-int zplane_groups(const BoxGeom& geo, int nstates) {
-  // about 2048 blocks (z-planes x groups) when every group gets 16 states
-  // or more; with fewer states, fewer groups down to about 512 blocks, each
-  // group then taking several states (one state per block repeats the
-  // block's set-up for little work)
-  const int hi = (2048 + geo.nz - 1) / geo.nz, lo = (512 + geo.nz - 1) / geo.nz;
-  int G = nstates / 16;
-  if (G > hi) G = hi;
-  if (G < lo) G = lo;
-  if (G > nstates) G = nstates;
-  return G < 1 ? 1 : G;
+// State groups of a z-plane pass: nz x G blocks, each with a run of states.
+// The G of the least expected time,
+//   blocks run by the busiest CU x states of the fullest group
+//     x (1 + tail / blocks per CU) x (1 + setup / states per block),
+// over at most max_blocks blocks: a number of blocks just below a multiple
+// of the 256 CUs and a G that divides the states well, more and shorter
+// blocks to even out the end of the pass, fewer to set up less (twiddles,
+// row indices; density: a partial plane written per block).  A CU is not
+// taken to be done faster with fewer blocks than `resident`.  Against fixed
+// targets of 512 .. 2048 blocks with 16 states each (us, density + vpsi,
+// before -> with this rule): 48^3, 112 states 127 -> 94; 60^3, 128 states
+// 269 -> 168; 75^3, 1984 states 6180 -> 5750; 64^3, 2048 states 2350 -> 2230;
+// 128^3, 128 states 1570 -> 1480.
+struct GroupWeights {
+  int max_blocks, resident;
+  double tail, setup;
+};
+static int zplane_groups(const BoxGeom& geo, int nstates,
+                         const GroupWeights& w) {
+  constexpr int kCUs = 256;
+  int most = w.max_blocks / geo.nz, best = 1;
+  if (most > nstates) most = nstates;
+  double least = 0;
+  for (int G = 1; G <= most; ++G) {
+    int rounds = (geo.nz * G + kCUs - 1) / kCUs;
+    if (rounds < w.resident) rounds = w.resident;
+    const int per = (nstates + G - 1) / G;
+    const double cost =
+        (double)rounds * per * (1 + w.tail / rounds) * (1 + w.setup / per);
+    if (G == 1 || cost < least) {
+      least = cost;
+      best = G;
+    }
+  }
+  return best;
+}
+
+// Passes of up to 4 waves a block (several blocks a CU): weights fitted to
+// the times at 22 sizes of 32 to 80 points and 64 to 1984 states, every G up
+// to 2304 blocks; on average within 2.2 % (density) and 1.4 % (vpsi) of the
+// best G.  8 waves a block (128 points, wide masks of 64) fill a CU by one
+// block, two in the density pass of 64 points: then as few blocks as keep
+// the CUs full are best (128^3, 128 states, density: 545 us with 2 groups,
+// 575 with 8, 621 with 16), and no tail shows.
+static bool wide_blocks(const BoxGeom& geo) {
+  return geo.nx == 128 || (geo.nx == 64 && z_window(geo) != 2);
+}
+int zplane_density_groups(const BoxGeom& geo, int nstates) {
+  return zplane_groups(geo, nstates,
+                       wide_blocks(geo)
+                           ? GroupWeights{2048, geo.nx == 64 ? 2 : 1, 0.0, 2.0}
+                           : GroupWeights{2048, 1, 0.25, 0.4});
+}
+int zplane_vpsi_groups(const BoxGeom& geo, int nstates) {
+  return zplane_groups(geo, nstates,
+                       wide_blocks(geo) ? GroupWeights{2048, 1, 0.0, 0.3}
+                                        : GroupWeights{3072, 1, 1.5, 0.4});
 }
 
 int launch_row_ifft(const double2* q, double2* R, int64_t state0, int nstates,

@@ -159,3 +159,17 @@ def test_row_path_128_mask_beyond_the_window():
   for k in ("w_re", "w_im"):
     g = r["d" + k].cpu().numpy()
     assert np.max(np.abs(g - grad[k])) < 1e-7 * np.max(np.abs(grad[k]))
+
+
+@pytest.mark.parametrize("n,nb,chunk", ((32, 15, 9), (48, 11, 6), (64, 9, 5),
+                                        (32, 4, 1)))
+def test_last_chunk_with_more_groups(n, nb, chunk):
+  """A shorter last chunk of states for which more state groups would be
+  best than the partial densities of the full chunks have room for (9 states
+  of 32^3: 5 groups, the last 6: 6 groups), against one sweep of all
+  states by the plane kernels."""
+  mask = _mask(n, n // 4)
+  path, a = _run(n, mask, 1, nb, band=True, chunk_states=chunk)
+  assert path
+  _, b = _run(n, mask, 1, nb, band=True, fft_variant=1)
+  _close(a, b)

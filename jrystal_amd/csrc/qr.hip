@@ -26,9 +26,12 @@ GramSplit gram_split(int64_t P, int ng, int nb) {
   int64_t want = (target + P - 1) / P;  // chunks per problem
   if (want < 1) want = 1;
   if (want > tiles) want = tiles;
-  const int tiles_per_chunk = (int)((tiles + want - 1) / want);
+  // whole 64-row tiles; for the wide kernels whole 16-row slabs, so that one
+  // block a CU leaves no CU without (137 059 rows: 252 blocks instead of 238)
+  const int unit = nb > kNarrowBands ? 16 : kQrRows;
+  const int units = (ng + unit - 1) / unit;
   GramSplit sp;
-  sp.rows_per_chunk = tiles_per_chunk * kQrRows;
+  sp.rows_per_chunk = (int)((units + want - 1) / want) * unit;
   sp.nchunk = (ng + sp.rows_per_chunk - 1) / sp.rows_per_chunk;
   return sp;
 }
@@ -113,7 +116,8 @@ __global__ __launch_bounds__(gram_wide_block(T)) void gram_wide_kernel(
   bool live[PW];
 #pragma unroll
   for (int t = 0; t < PW; ++t) {
-    const int q = ((int)blockIdx.z * PL::NW + wave) * PW + t;
+    // dealt round: waves w and w + 4 share a SIMD, 9 of 36 pairs to each
+    const int q = (t * PL::NZ + (int)blockIdx.z) * PL::NW + wave;
     live[t] = q < PL::NPAIR;  // uniform over the wave
     decode_pair(live[t] ? q : 0, T, HERM, &pI[t], &pJ[t]);
   }
@@ -245,133 +249,182 @@ int launch_gram_wide(const double* wr, const double* wi, const double2* qa,
 }
 
 constexpr int kWideRows = 64;  // g rows per block of the wide apply kernels
-constexpr int kWideK = 32;     // rinv rows per LDS chunk (apply_fwd)
-constexpr int kWideKB = 16;    // band rows per LDS chunk (apply_bwd)
 
-// apply_fwd_kernel for nb > 64: rinv staged in chunks of kWideK rows, one
-// 16-row slab of W per wave; tiles below the diagonal of rinv are skipped.
+// apply_fwd_kernel for nb > 64.  One 16-row slab of W per wave; rinv is
+// staged in LDS by chunks of 16 rows (the tiles on and right of the
+// diagonal), double-buffered: the next chunk of rinv and of the wave's W
+// is in flight in registers while the MFMAs run on the current one.  The
+// chunks are unrolled, so that the triangular tile loop has no branch (a
+// branch costs copies of the accumulators, which wait for the matrix unit).
+// k of an MFMA step is 16 c + 4 lk + m: a lane's four W values are adjacent.
+// FP64 MFMA bound: 137 059 x 128: 340 us before (43 % MFMA
+// busy), 210 now (67 %).
 template <int T>
 __global__ __launch_bounds__(kQrBlock) void apply_fwd_wide_kernel(
     const double* __restrict__ wr, const double* __restrict__ wi,
     const double2* __restrict__ rinv, double2* __restrict__ q, int ng, int nb,
     const int* __restrict__ skip) {
-  extern __shared__ double2 sm[];  // [kWideK][NBP]
+  extern __shared__ double2 sm[];  // [2][16][NBP]
   constexpr int NBP = 16 * T;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
+  const int sk = threadIdx.x >> 4, sj = threadIdx.x & 15;  // staged element
   const int64_t p = blockIdx.y;
   if (skip && skip[p]) return;  // uniform over the block
   const double2* Rp = rinv + p * nb * nb;
-  const double* Wr = wr + p * ng * nb;
-  const double* Wi = wi + p * ng * nb;
-  double2* Q = q + p * nb * ng;
   const int g0 = blockIdx.x * kWideRows + wave * 16;
   const int row = g0 + li;
+  const double* Wr = wr + (p * ng + row) * nb;
+  const double* Wi = wi + (p * ng + row) * nb;
+  double2* Q = q + p * nb * ng;
+  double2 st[T];
+  double ar[2][4], ai[2][4];
+  auto fetch = [&](int c, double (&xr)[4], double (&xi)[4]) {
+    const int k = 16 * c + sk;
+#pragma unroll
+    for (int J = c; J < T; ++J) {
+      const int b = 16 * J + sj;
+      st[J] = (k < nb && b < nb) ? Rp[k * nb + b] : czero();
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int col = 16 * c + 4 * lk + m;
+      const bool ok = row < ng && (c < T - 1 || col < nb);
+      xr[m] = ok ? Wr[col] : 0.0;
+      xi[m] = ok ? Wi[col] : 0.0;
+    }
+  };
   d4 qre[T], qim[T];
 #pragma unroll
   for (int J = 0; J < T; ++J) { qre[J] = d4zero(); qim[J] = d4zero(); }
-  for (int k0 = 0; k0 < nb; k0 += kWideK) {
-    __syncthreads();  // the previous chunk is consumed
-    for (int e = threadIdx.x; e < kWideK * NBP; e += kQrBlock) {
-      const int kk = e / NBP, b = e - kk * NBP, k = k0 + kk;
-      sm[e] = (k < nb && b < nb) ? Rp[k * nb + b] : czero();
-    }
-    __syncthreads();
-#pragma unroll 2
-    for (int m = 0; m < kWideK / 4; ++m) {
-      const int col = k0 + 4 * m + lk;
-      const bool ok = row < ng && col < nb;
-      const double a_r = ok ? Wr[(int64_t)row * nb + col] : 0.0;
-      const double a_i = ok ? Wi[(int64_t)row * nb + col] : 0.0;
+  fetch(0, ar[0], ai[0]);
 #pragma unroll
-      for (int J = 0; J < T; ++J) {
-        if (16 * J + 15 < k0) continue;  // rinv[k][b] = 0 for k > b
-        const double2 rv = sm[(4 * m + lk) * NBP + 16 * J + li];
+  for (int c = 0; c < T; ++c) {
+    double2* buf = sm + (c & 1) * 16 * NBP;
+    // (buffer c & 1 was last read before the barrier of chunk c - 1)
+#pragma unroll
+    for (int J = c; J < T; ++J) buf[sk * NBP + 16 * J + sj] = st[J];
+    __syncthreads();
+    if (c + 1 < T) fetch(c + 1, ar[(c + 1) & 1], ai[(c + 1) & 1]);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const double a_r = ar[c & 1][m], a_i = ai[c & 1][m];
+#pragma unroll
+      for (int J = c; J < T; ++J) {  // rinv[k][b] = 0 for k > b
+        const double2 rv = buf[(4 * lk + m) * NBP + 16 * J + li];
         qre[J] = mfma4(rv.x, a_r, qre[J]);
-        qre[J] = mfma4(-rv.y, a_i, qre[J]);
         qim[J] = mfma4(rv.x, a_i, qim[J]);
+        qre[J] = mfma4(-rv.y, a_i, qre[J]);
         qim[J] = mfma4(rv.y, a_r, qim[J]);
       }
     }
   }
+  if (row >= ng) return;
 #pragma unroll
   for (int J = 0; J < T; ++J)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int b = 16 * J + 4 * r + lk;
-      if (b < nb && row < ng)
+      if (J < T - 1 || b < nb)
         Q[(int64_t)b * ng + row] = make_double2(qre[J][r], qim[J][r]);
     }
 }
 
-// apply_bwd_kernel for nb > 64: A and Bm staged in chunks of kWideKB band
-// rows, one 16-row slab of the output per wave; A = rinv^H is lower
-// triangular, so its tiles right of the chunk are skipped.
+// apply_bwd_kernel for nb > 64.  As apply_fwd_wide_kernel, with A (lower
+// triangular: the tiles left of and on the diagonal) and Bm staged side by
+// side; two waves share a 16-row slab, one the even and one the odd column
+// tiles (an even and an odd wave to each SIMD), so that a block of eight
+// waves, whose LDS fills a CU, still takes only 64 rows (137 059 rows are
+// 8.4 such blocks a CU).
+// FP64 MFMA bound: 137 059 x 128: 678 us before (57 % MFMA
+// busy), 535 now (73 %).
+constexpr int kWideBwdBlock = 512;
 template <int T>
-__global__ __launch_bounds__(kQrBlock) void apply_bwd_wide_kernel(
+__global__ __launch_bounds__(kWideBwdBlock) void apply_bwd_wide_kernel(
     const double2* __restrict__ qbar, const double2* __restrict__ q,
     const double2* __restrict__ A, const double2* __restrict__ Bm,
     double* __restrict__ dwr, double* __restrict__ dwi, int ng, int nb) {
-  extern __shared__ double2 sm[];
-  constexpr int NBP = 16 * T;
-  double2* sa = sm;                   // [kWideKB][NBP]
-  double2* sb = sm + kWideKB * NBP;   // [kWideKB][NBP]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
+  extern __shared__ double2 sm[];  // [2][2][16][NBP]
+  constexpr int NBP = 16 * T, TH = (T + 1) / 2;
+  // (the wave index through readfirstlane: branches on it are scalar)
+  const int lane = threadIdx.x & 63,
+            wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lk = lane >> 4, odd = (wave ^ (wave >> 2)) & 1;
+  const int sk = (threadIdx.x >> 4) & 15, sj = threadIdx.x & 15;
+  const int mat = wave >> 2;  // staged matrix: 0 = A, 1 = Bm
   const int64_t p = blockIdx.y;
-  const double2* Ap = A + p * nb * nb;
-  const double2* Bp = Bm + p * nb * nb;
-  const double2* Qb = qbar + p * nb * ng;
-  const double2* Q = q + p * nb * ng;
+  const double2* Sp = (mat ? Bm : A) + p * nb * nb;
+  const int g0 = blockIdx.x * kWideRows + (wave >> 1) * 16;
+  const int g = g0 + li;
+  const double2* Qb = qbar + p * nb * ng + g;
+  const double2* Q = q + p * nb * ng + g;
   double* Dr = dwr + p * ng * nb;
   double* Di = dwi + p * ng * nb;
-  const int g0 = blockIdx.x * kWideRows + wave * 16;
-  const int g = g0 + li;
-  d4 re[T], im[T];
+  double2 st[T], vb[2][4], vq[2][4];
+  auto fetch = [&](int c, double2 (&xb)[4], double2 (&xq)[4]) {
+    const int k = 16 * c + sk;
 #pragma unroll
-  for (int J = 0; J < T; ++J) { re[J] = d4zero(); im[J] = d4zero(); }
-  for (int k0 = 0; k0 < nb; k0 += kWideKB) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < kWideKB * NBP; e += kQrBlock) {
-      const int kk = e / NBP, b = e - kk * NBP, k = k0 + kk;
-      const bool ok = k < nb && b < nb;
-      sa[e] = ok ? Ap[k * nb + b] : czero();
-      sb[e] = ok ? Bp[k * nb + b] : czero();
+    for (int J = 0; J < T; ++J) {
+      const int b = 16 * J + sj;
+      st[J] = (k < nb && b < nb && (J <= c || mat)) ? Sp[k * nb + b] : czero();
     }
-    __syncthreads();
-#pragma unroll 2
-    for (int m = 0; m < kWideKB / 4; ++m) {
-      const int band = k0 + 4 * m + lk;
-      const bool ok = g < ng && band < nb;
-      const double2 vb = ok ? Qb[(int64_t)band * ng + g] : czero();
-      const double2 vq = ok ? Q[(int64_t)band * ng + g] : czero();
 #pragma unroll
-      for (int J = 0; J < T; ++J) {
-        if (16 * J < k0 + kWideKB) {  // A[i][j] = 0 for j > i
-          const double2 a = sa[(4 * m + lk) * NBP + 16 * J + li];
-          re[J] = mfma4(vb.x, a.x, re[J]);
-          re[J] = mfma4(-vb.y, a.y, re[J]);
-          im[J] = mfma4(vb.x, a.y, im[J]);
-          im[J] = mfma4(vb.y, a.x, im[J]);
+    for (int m = 0; m < 4; ++m) {
+      const int band = 16 * c + 4 * m + lk;
+      const bool ok = g < ng && (c < T - 1 || band < nb);
+      xb[m] = ok ? Qb[(int64_t)band * ng] : czero();
+      xq[m] = ok ? Q[(int64_t)band * ng] : czero();
+    }
+  };
+  d4 re[TH], im[TH];
+#pragma unroll
+  for (int h = 0; h < TH; ++h) { re[h] = d4zero(); im[h] = d4zero(); }
+  fetch(0, vb[0], vq[0]);
+#pragma unroll
+  for (int c = 0; c < T; ++c) {
+    double2* buf = sm + (c & 1) * 2 * 16 * NBP;
+    // (buffer c & 1 was last read before the barrier of chunk c - 1)
+#pragma unroll
+    for (int J = 0; J < T; ++J)
+      if (J <= c || mat) buf[(mat * 16 + sk) * NBP + 16 * J + sj] = st[J];
+    __syncthreads();
+    if (c + 1 < T) fetch(c + 1, vb[(c + 1) & 1], vq[(c + 1) & 1]);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const double2 xb = vb[c & 1][m], xq = vq[c & 1][m];
+      const double2* sa = buf + (4 * m + lk) * NBP + 16 * odd + li;
+      const double2* sb = sa + 16 * NBP;
+#pragma unroll
+      for (int h = 0; h < TH; ++h) {  // column tile 2 h + odd
+        if (2 * h + 1 <= c || (2 * h <= c && !odd)) {  // A[i][j] = 0 for j > i
+          const double2 a = sa[32 * h];
+          re[h] = mfma4(xb.x, a.x, re[h]);
+          im[h] = mfma4(xb.x, a.y, im[h]);
+          re[h] = mfma4(-xb.y, a.y, re[h]);
+          im[h] = mfma4(xb.y, a.x, im[h]);
         }
-        const double2 b = sb[(4 * m + lk) * NBP + 16 * J + li];
-        re[J] = mfma4(vq.x, b.x, re[J]);
-        re[J] = mfma4(-vq.y, b.y, re[J]);
-        im[J] = mfma4(vq.x, b.y, im[J]);
-        im[J] = mfma4(vq.y, b.x, im[J]);
+        if (2 * h + 1 < T || !odd) {
+          const double2 b = sb[32 * h];
+          re[h] = mfma4(xq.x, b.x, re[h]);
+          im[h] = mfma4(xq.x, b.y, im[h]);
+          re[h] = mfma4(-xq.y, b.y, re[h]);
+          im[h] = mfma4(xq.y, b.x, im[h]);
+        }
       }
     }
   }
 #pragma unroll
-  for (int J = 0; J < T; ++J)
+  for (int h = 0; h < TH; ++h) {
+    const int col = 16 * (2 * h + odd) + li;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = g0 + 4 * r + lk, col = 16 * J + li;
+      const int row = g0 + 4 * r + lk;
       if (row < ng && col < nb) {
-        Dr[(int64_t)row * nb + col] = re[J][r];
-        Di[(int64_t)row * nb + col] = im[J][r];
+        Dr[(int64_t)row * nb + col] = re[h][r];
+        Di[(int64_t)row * nb + col] = im[h][r];
       }
     }
+  }
 }
 
 // Partial Gram sums over the chunk's rows (one per block):
@@ -821,7 +874,7 @@ int launch_apply_fwd(const double* wr, const double* wi, const double2* rinv,
                      const int* skip) {
   const int T = (nb + 15) / 16;
   if (nb > kNarrowBands) {
-    const size_t shm = (size_t)kWideK * 16 * T * sizeof(double2);
+    const size_t shm = 2 * (size_t)16 * 16 * T * sizeof(double2);
     dim3 grid(ceil_div(ng, kWideRows), (unsigned)P), block(kQrBlock);
     switch (T) {
       case 5: hipLaunchKernelGGL((apply_fwd_wide_kernel<5>), grid, block, shm, s, wr, wi, rinv, q, ng, nb, skip); break;
@@ -950,8 +1003,8 @@ size_t qr_lds_bytes(int nb) {
   if (nb <= kNarrowBands)  // Gram (pre + sums), apply_bwd
     return std::max(2 * nbp * nbp * z, chol);
   const size_t gram = 2 * 2 * (size_t)wide_slab<false>() * (nbp + 1) * z;
-  const size_t fwd = (size_t)kWideK * nbp * z;
-  const size_t bwd = 2 * (size_t)kWideKB * nbp * z;
+  const size_t fwd = 2 * (size_t)16 * nbp * z;
+  const size_t bwd = 2 * fwd;
   return std::max(std::max(gram, fwd), std::max(bwd, chol));
 }
 
@@ -960,8 +1013,8 @@ int launch_apply_bwd(const double2* qbar, const double2* q, const double2* A,
                      int ng, int nb, hipStream_t s) {
   const int T = (nb + 15) / 16;
   if (nb > kNarrowBands) {
-    const size_t shm = 2 * (size_t)kWideKB * 16 * T * sizeof(double2);
-    dim3 grid(ceil_div(ng, kWideRows), (unsigned)P), block(kQrBlock);
+    const size_t shm = 2 * 2 * (size_t)16 * 16 * T * sizeof(double2);
+    dim3 grid(ceil_div(ng, kWideRows), (unsigned)P), block(kWideBwdBlock);
     switch (T) {
       case 5: hipLaunchKernelGGL((apply_bwd_wide_kernel<5>), grid, block, shm, s, qbar, q, A, Bm, dwr, dwi, ng, nb); break;
       case 6: hipLaunchKernelGGL((apply_bwd_wide_kernel<6>), grid, block, shm, s, qbar, q, A, Bm, dwr, dwi, ng, nb); break;

@@ -19,7 +19,7 @@ constexpr int kNarrowBands = 64;
 constexpr int kMaxBands = 128;
 
 struct GramSplit {
-  int rows_per_chunk;  // multiple of kQrRows
+  int rows_per_chunk;  // multiple of kQrRows (wide kernels: of 16)
   int nchunk;          // chunks per problem
 };
 GramSplit gram_split(int64_t P, int ng, int nb);

@@ -7,30 +7,37 @@
 namespace jrx {
 namespace {
 
-constexpr int kFwdBlock = 256;
 constexpr int kBwdTile = 128;      // samples per backward tile (one per thread)
 constexpr int kBwdStride = kBwdTile + 1;  // padded LDS rows
 constexpr int kBwdMaxBlocks = 1024;
 constexpr int kLossBlock = 256;
 
-__global__ void __launch_bounds__(kFwdBlock)
+__global__ void __launch_bounds__(kMlpBlock, 4)
 mlp_forward_kernel(const float* __restrict__ params,
                    const float* __restrict__ norm,
                    const float* __restrict__ x, int64_t n,
                    float* __restrict__ y) {
-  __shared__ float w[kMlpParams];
-  mlp_stage(params, w);
+  __shared__ f4 w[MlpWave::kF4];
+  __shared__ float xs[kMlpBlock * MlpWave::kRow];
+  const int lane = threadIdx.x & 63;
+  float* xw = xs + (threadIdx.x - lane) * MlpWave::kRow;
+  MlpWave net;
+  net.load(params, w, lane);
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * kFwdBlock + threadIdx.x;
-  if (i >= n) return;
-  float xi[kMlpIn];
+  int64_t end;
+  for (int64_t i0 = mlp_run(n, &end); i0 < end; i0 += 64) {
+    const int64_t i = i0 + lane;
+    float xi[kMlpIn];
 #pragma unroll
-  for (int k = 0; k < kMlpIn; ++k) xi[k] = x[i * kMlpIn + k];
-  mlp_normalise(norm, xi);
-  float yi[kMlpOut];
-  mlp_eval(w, xi, yi);
-  y[i * kMlpOut] = yi[0];
-  y[i * kMlpOut + 1] = yi[1];
+    for (int k = 0; k < kMlpIn; ++k) xi[k] = i < n ? x[i * kMlpIn + k] : 0.f;
+    mlp_normalise(norm, xi);
+    float yi[kMlpOut];
+    net.eval(xi, xw, lane, yi);
+    if (i < n) {
+      y[i * kMlpOut] = yi[0];
+      y[i * kMlpOut + 1] = yi[1];
+    }
+  }
 }
 
 // Parameter gradient of sum_i dy_i . y(x_i).  Block b takes tiles b,
@@ -246,8 +253,8 @@ int jrx_mlp_forward(const float* params, const float* norm, const float* x,
                     int64_t n, float* y, void* stream) {
   JRX_REQUIRE(params && norm && x && y && n >= 0, "invalid mlp arguments");
   if (n == 0) return JRX_OK;
-  hipLaunchKernelGGL(mlp_forward_kernel, dim3(ceil_div(n, kFwdBlock)),
-                     dim3(kFwdBlock), 0, (hipStream_t)stream, params, norm, x,
+  hipLaunchKernelGGL(mlp_forward_kernel, dim3(mlp_blocks(n)),
+                     dim3(kMlpBlock), 0, (hipStream_t)stream, params, norm, x,
                      n, y);
   JRX_LAUNCH_CHECK();
   return JRX_OK;

@@ -958,7 +958,7 @@ __global__ void coef_features_kernel(const int64_t* __restrict__ idx,
 
 // Network inference on every coefficient: factor[i] = exp(y0) and, when
 // w is given, w[i] *= exp(y1) (warm start), y clamped before exp.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kMlpBlock, 4)
 coef_mlp_kernel(const float* __restrict__ params,
                 const float* __restrict__ norm, int64_t n,
                 const double* __restrict__ tb, const short* __restrict__ g_m,
@@ -967,30 +967,52 @@ coef_mlp_kernel(const float* __restrict__ params,
                 const double* __restrict__ gap,
                 double* __restrict__ factor, double* __restrict__ wr,
                 double* __restrict__ wi) {
-  __shared__ float w[kMlpParams];
-  mlp_stage(params, w);
+  __shared__ f4 w[MlpWave::kF4];
+  __shared__ float xs[kMlpBlock * MlpWave::kRow];
+  const int lane = threadIdx.x & 63;
+  float* xw = xs + (threadIdx.x - lane) * MlpWave::kRow;
+  MlpWave net;
+  net.load(params, w, lane);
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int b = (int)(i % nb);
-  const int64_t rest = i / nb;
-  const int g = (int)(rest % ng);
-  const int64_t sk = rest / ng;
-  const int k = (int)(sk % nk);
-  float f[kMlpIn];
-  const int64_t st = sk * nb + b;
-  mlp_features(coef_gk2(g_m, kpts, cp, g, k), tb[st], gap ? gap[st] : 0.0,
-               stats[0], stats[1], f);
-  mlp_normalise(norm, f);
-  float y[kMlpOut];
-  mlp_eval(w, f, y);
-  if (factor)
-    factor[i] = exp((double)fminf(fmaxf(y[0], kLogFactorMin), kLogFactorMax));
-  if (wr) {
-    const double a =
-        exp((double)fminf(fmaxf(y[1], kLogAmpMin), kLogAmpMax));
-    wr[i] *= a;
-    wi[i] *= a;
+  // features of the density and, while it stays the same, of the state
+  float fs[kMlpIn] = {};
+  mlp_density_features(stats[0], stats[1], fs);
+  int64_t state = -1;
+  double t = 0.0;
+  int64_t end;
+  for (int64_t i0 = mlp_run(n, &end); i0 < end; i0 += 64) {
+    const int64_t i = i0 + lane;
+    float f[kMlpIn] = {};
+    if (i < n) {
+      // 64-bit divisions for the wave's first coefficient only
+      const int64_t rest = i0 / nb, sk0 = rest / ng;
+      const unsigned ub = (unsigned)(i0 - rest * nb) + lane;
+      const unsigned ug = (unsigned)(rest - sk0 * ng) + ub / nb;
+      const int b = (int)(ub % nb), g = (int)(ug % ng);
+      const int64_t sk = sk0 + ug / ng;
+      const int64_t st = sk * nb + b;
+      if (st != state) {
+        state = st;
+        t = tb[st];
+        mlp_state_features(t, gap ? gap[st] : 0.0, fs);
+      }
+#pragma unroll
+      for (int j = 0; j < kMlpIn; ++j) f[j] = fs[j];
+      mlp_plane_wave_features(
+          coef_gk2(g_m, kpts, cp, g, (int)((unsigned)sk % nk)), t, f);
+    }
+    mlp_normalise(norm, f);
+    float y[kMlpOut];
+    net.eval(f, xw, lane, y);
+    if (i >= n) continue;
+    if (factor)
+      factor[i] = exp((double)fminf(fmaxf(y[0], kLogFactorMin), kLogFactorMax));
+    if (wr) {
+      const double a =
+          exp((double)fminf(fmaxf(y[1], kLogAmpMin), kLogAmpMax));
+      wr[i] *= a;
+      wi[i] *= a;
+    }
   }
 }
 
@@ -1047,7 +1069,7 @@ extern "C" int jrx_plan_mlp_apply(const jrx_plan* p, const float* params,
   const int64_t n = p->S * p->ng;
   const double* tb = reinterpret_cast<const double*>(
       static_cast<const char*>(workspace) + p->o_tb);
-  hipLaunchKernelGGL(coef_mlp_kernel, dim3(ceil_div(n, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(coef_mlp_kernel, dim3(mlp_blocks(n)), dim3(kMlpBlock), 0,
                      (hipStream_t)stream, params, norm, n, tb, p->d_g_m,
                      p->d_kpts, p->cp, p->ng, p->nk, p->nb, stats, gap,
                      factor, w_re, w_im);

@@ -281,3 +281,35 @@ def test_fallback_to_plain_preconditioner():
   e = [h[1] for h in r.history]
   assert all(np.isfinite(e))
   assert all(b <= a + 1e-12 for a, b in zip(e, e[1:]))
+
+
+@pytest.mark.parametrize("n", (1, 15, 64, 65, 257, 4 * 65536 + 70))
+def test_mlp_forward_of_ragged_sizes(n):
+  """Parts of a 16-sample tile, of a wave's 64 and of a block, and more
+  samples than one run per wave, against the network in 64 bits."""
+  L = _lib()
+  rng, p, norm = _net(3)
+  x = (rng.standard_normal((n, 8)) * 2).astype(np.float32)
+  pt, nt, xt = _dev(p), _dev(norm), _dev(x)
+  y = torch.full((n + 1, 2), 7.0, dtype=torch.float32, device="cuda")
+  L.check(L.lib().jrx_mlp_forward(pt.data_ptr(), nt.data_ptr(), xt.data_ptr(),
+                                  n, y.data_ptr(), L.stream_ptr()))
+  assert (y[n] == 7.0).all()  # nothing past the last sample
+  P, nm = p.astype(np.float64), norm.astype(np.float64)
+  w1, b1 = P[:512].reshape(64, 8), P[512:576]
+  w2, b2 = P[576:4672].reshape(64, 64), P[4672:4736]
+  w3, b3 = P[4736:4864].reshape(2, 64), P[4864:4866]
+  xn = (x - nm[:8]) * nm[8:]
+  h1 = np.tanh(xn @ w1.T + b1)
+  h2 = np.tanh(h1 @ w2.T + b2)
+  ref = h2 @ w3.T + b3
+  # FP32 bounds, u = 2^-24: a sum of K terms adds K u sum |w h|, tanh (of
+  # slope <= 1) 4 u, the normalisation 2 u of (|x| + |mu|) / sd
+  u = 2.0**-24
+  e0 = 3 * u * (np.abs(x) + np.abs(nm[:8])) * nm[8:]
+  e1 = e0 @ np.abs(w1).T + 10 * u * (np.abs(xn) @ np.abs(w1).T +
+                                     np.abs(b1)) + 4 * u
+  e2 = e1 @ np.abs(w2).T + 66 * u * (np.abs(h1) @ np.abs(w2).T +
+                                     np.abs(b2)) + 4 * u
+  ey = e2 @ np.abs(w3).T + 66 * u * (np.abs(h2) @ np.abs(w3).T + np.abs(b3))
+  assert (np.abs(y[:n].cpu().numpy() - ref) <= ey).all()

@@ -159,11 +159,20 @@ static int zplane_groups(const BoxGeom& geo, int nstates,
 static bool wide_blocks(const BoxGeom& geo) {
   return geo.nx == 128 || (geo.nx == 64 && z_window(geo) != 2);
 }
+// The partial planes are part of the workspace.  64 and 128 points gain
+// nothing from more groups than one per 16 states above 512 blocks (64^3, 64
+// states: 8 groups 41 us, 16 groups 44 us), so they stay within that.
 int zplane_density_groups(const BoxGeom& geo, int nstates) {
+  const bool wide = wide_blocks(geo);
+  int most = 2048;
+  if (geo.nx == 64 || geo.nx == 128) {
+    const int few = (512 + geo.nz - 1) / geo.nz;
+    most = geo.nz * (nstates / 16 > few ? nstates / 16 : few);
+    if (most > 2048) most = 2048;
+  }
   return zplane_groups(geo, nstates,
-                       wide_blocks(geo)
-                           ? GroupWeights{2048, geo.nx == 64 ? 2 : 1, 0.0, 2.0}
-                           : GroupWeights{2048, 1, 0.25, 0.4});
+                       wide ? GroupWeights{most, geo.nx == 64 ? 2 : 1, 0.0, 2.0}
+                            : GroupWeights{most, 1, 0.25, 0.4});
 }
 int zplane_vpsi_groups(const BoxGeom& geo, int nstates) {
   return zplane_groups(geo, nstates,

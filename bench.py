@@ -753,10 +753,10 @@ KERNEL_NAMES = {"xline_vpsi": "jrx::xline_vpsi64_kernel",
                 "plane_ifft": "jrx::plane_ifft64_kernel",
                 "xline_density": "jrx::xline_density64_kernel",
                 "plane_fft_gather": "jrx::plane_fft_gather64_kernel",
-                "zplane_vpsi": "jrx::zplane_vpsi_kernel<64, 1, 256>",
-                "row_ifft": "jrx::row_ifft_kernel<64>",
-                "zplane_density": "jrx::zplane_density_kernel<64, 1, 256>",
-                "row_fft_gather": "jrx::row_fft_gather_kernel<64, false>"}
+                "zplane_vpsi": "jrx::zplane_vpsi_kernel<64, 2, 4, true, true>",
+                "row_ifft": "jrx::row_ifft_kernel<64, 2>",
+                "zplane_density": "jrx::zplane_density_kernel<64, 2, 4, true>",
+                "row_fft_gather": "jrx::row_fft_gather_kernel<64, 2, false>"}
 # On the row-buffer path the four FFT timing classes hold these kernels.
 ROW_PATH_CLASSES = {"plane_ifft": "row_ifft",
                     "xline_density": "zplane_density",

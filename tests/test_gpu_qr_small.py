@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from jrystal_amd import _lib, _ops
+from jrystal_amd.objective import EnergyPlan
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +73,29 @@ def test_dependent_columns_give_nan(nb):
   _lib.check(L.jrx_qr(wr.data_ptr(), wi.data_ptr(), 1, ng, nb, q.data_ptr(),
                       ri.data_ptr(), wp, ws.numel() - 256, _lib.stream_ptr()))
   assert torch.isnan(torch.view_as_real(q)).any()
+
+
+@pytest.mark.parametrize("nb", (1, 16, 17, 32, 33, 48, 64, 65, 100, 128))
+def test_one_pass_columns_have_unit_norm(nb):
+  """Rounding of the pivots' inverse square roots alone: columns with one
+  nonzero entry c each have an exactly diagonal Gram matrix, so that the
+  adaptive QR takes one pass and |Q| = |c| / sqrt(fl(c^2)).  With u = 2^-53:
+  half of the square's u, 1.25 u of the root (1.4e-16) and u of the product
+  make less than 3 u."""
+  f = np.arange(16)
+  f = np.where(f < 8, f, f - 16)
+  mask = f[:, None, None]**2 + f[:, None]**2 + f**2 <= 21
+  ng, nk = int(mask.sum()), 8
+  plan = EnergyPlan(np.zeros((1, 3)), np.array([4.0]), 8.0 * np.eye(3), mask,
+                    np.zeros((nk, 3)), np.ones((1, nk, nb)))
+  rng = np.random.default_rng(nb)
+  c = np.exp(rng.uniform(-20.0, 20.0, (nk, nb)))
+  rows = np.stack([rng.permutation(ng)[:nb] for _ in range(nk)])
+  w = np.zeros((1, nk, ng, nb))
+  np.put_along_axis(w[0], rows[:, None], c[:, None], axis=1)
+  w = torch.tensor(w, device="cuda")
+  plan.evaluate(w, torch.zeros_like(w), grad=False)
+  q = plan.orthonormal_params()[0].cpu().numpy()[0]
+  got = np.take_along_axis(q, rows[:, None], axis=1)[:, 0]
+  assert np.count_nonzero(q) == nk * nb
+  assert np.max(np.abs(got - 1)) <= 3 * 2.0**-53

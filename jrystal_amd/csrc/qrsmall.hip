@@ -87,15 +87,18 @@ __device__ __forceinline__ double lane_value(double v) {
 // Step S of the elimination of a 16 x 16 Hermitian positive tile on one
 // wave: lane l holds row r = l % 16, columns 4 (l / 16) + q of A and of
 // E = (product of the elimination steps).  f_r = A[r][S] / A[S][S] for the
-// rows below; the rows' 1 / sqrt(pivot) collect in ysr.
+// rows below; the rows' 1 / sqrt(pivot) collect in ysr.  n: rows of the tile
+// inside the matrix (from row n on it is the identity, which no step changes:
+// jrx_qr, 8 problems of 2000 rows, 1 band: 26.7 us with all 16 steps, 21.5).
 template <int S>
 __device__ __forceinline__ void chol_step(double2 (&a)[4], double2 (&e)[4],
-                                          double& ysr, int r) {
+                                          double& ysr, int r, int n) {
   constexpr int K = S >> 2, Q = S & 3;
   const double piv = lane_value<S + 16 * K>(a[Q].x);
   const double ys = rsqrt_series(piv);
   if (r == S) ysr = ys;
   if constexpr (S < 15) {
+    if (S + 1 >= n) return;
     const double y = r > S ? ys : 0.0;
     const double2 f = make_double2(rows_bcast<K>(a[Q].x) * y * y,
                                    rows_bcast<K>(a[Q].y) * y * y);
@@ -108,11 +111,12 @@ __device__ __forceinline__ void chol_step(double2 (&a)[4], double2 (&e)[4],
       a[q] = csub(a[q], cmul(f, pa));
       e[q] = csub(e[q], cmul(f, pe));
     }
-    chol_step<S + 1>(a, e, ysr, r);
+    chol_step<S + 1>(a, e, ysr, r, n);
   }
 }
 // The tile (its factor R_dd aside) becomes X = R_dd^{-1} = E^H.
-__device__ __forceinline__ void chol_tile(double2* C, int lane) {
+__device__ __forceinline__ void chol_tile(double2* C, int lane,
+                                          int n) {
   const int r = lane & 15, g = lane >> 4;
   double2 a[4], e[4];
   double ysr = 1.0;
@@ -121,7 +125,7 @@ __device__ __forceinline__ void chol_tile(double2* C, int lane) {
     a[q] = C[tile_at(r, 4 * g + q)];
     e[q] = make_double2(r == 4 * g + q ? 1.0 : 0.0, 0.0);
   }
-  chol_step<0>(a, e, ysr, r);
+  chol_step<0>(a, e, ysr, r, n);
 #pragma unroll
   for (int q = 0; q < 4; ++q)
     C[tile_at(4 * g + q, r)] = make_double2(ysr * e[q].x, -ysr * e[q].y);
@@ -191,7 +195,7 @@ void chol_inv_kernel(const double2* __restrict__ S,
       flag_out[p] = (d2 < kQrOnePass * kQrOnePass) ? 1 : 0;
   }
   __syncthreads();
-  if (wave == 0) chol_tile(tile(0, 0), lane);
+  if (wave == 0) chol_tile(tile(0, 0), lane, nb);
   __syncthreads();
 #pragma unroll 1
   for (int d = 0; d + 1 < T; ++d) {
@@ -215,7 +219,7 @@ void chol_inv_kernel(const double2* __restrict__ S,
     if (wave == 0) {
       update(d + 1, d + 1);
       wave_order();
-      chol_tile(tile(d + 1, d + 1), lane);
+      chol_tile(tile(d + 1, d + 1), lane, nb - 16 * (d + 1));
     } else {
       int n = 0;  // the other tiles, dealt to the other waves
       for (int I = d + 1; I < T; ++I)

@@ -304,36 +304,48 @@ int launch_chol_inv(const double2* S, double2* rinv, int64_t P, int nb,
   return JRX_OK;
 }
 
-// A = R^{-H} and B = copyltu(triu(-G)) R^{-H}, one 16 x 16 tile per wave,
-// operands from global memory (L2): B_IJ = sum_{K >= J} M_IK (Ri_JK)^H, with
-// M[i][k] = -G[i][k] above the diagonal, its mirror image below and
-// -Re G[i][i] on it.
+// A = R^{-H} and B = copyltu(triu(-G)) R^{-H}, operands from global memory
+// (L2): B_IJ = sum_{K >= J} M_IK (Ri_JK)^H, with M[i][k] = -G[i][k] above the
+// diagonal, its mirror image below and -Re G[i][i] on it.  A_IJ = (Ri_JI)^H
+// is the operand of K = I.
+// Step s (of four in k) of the tiles (I, K) of M and (J, K) of Ri^H.
+__device__ __forceinline__ void adjoint_step(const double2* Gp,
+                                             const double2* Rp, int nb, int i,
+                                             int j, int k, double2& a,
+                                             double2& b) {
+  a = b = czero();
+  if (i < nb && k < nb) {
+    const double2 g = i <= k ? Gp[i * nb + k] : Gp[k * nb + i];
+    a = make_double2(-g.x, i < k ? -g.y : i > k ? g.y : 0.0);
+  }
+  if (j <= k && k < nb) b = cconj(Rp[j * nb + k]);
+}
+
+// One 16 x 16 tile per wave.
 __global__ __launch_bounds__(256) void qr_bwd_small_kernel(
     const double2* __restrict__ G, const double2* __restrict__ rinv,
     double2* __restrict__ A, double2* __restrict__ Bm, int nb, int T) {
   const int64_t p = blockIdx.y;
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t =
+      blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (t >= T * T) return;
   const int I = t / T, J = t - I * T;
   const double2* Gp = G + p * nb * nb;
   const double2* Rp = rinv + p * nb * nb;
   TileAcc c;
+  double2 aij[4] = {czero(), czero(), czero(), czero()};
   const int i = 16 * I + li, j = 16 * J + li;
   for (int K = J; K < T; ++K) {
     double2 a[4], b[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int k = 16 * K + 4 * s + lk;
-      a[s] = b[s] = czero();
-      if (i < nb && k < nb) {
-        const double2 g = i <= k ? Gp[i * nb + k] : Gp[k * nb + i];
-        a[s] = make_double2(-g.x, i < k ? -g.y : i > k ? g.y : 0.0);
-      }
-      if (j <= k && k < nb) b[s] = cconj(Rp[j * nb + k]);
-    }
+    for (int s = 0; s < 4; ++s)
+      adjoint_step(Gp, Rp, nb, i, j, 16 * K + 4 * s + lk, a[s], b[s]);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) c.step(a[s], b[s]);
+    for (int s = 0; s < 4; ++s) {
+      c.step(a[s], b[s]);
+      if (K == I) aij[s] = b[s];
+    }
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -341,17 +353,52 @@ __global__ __launch_bounds__(256) void qr_bwd_small_kernel(
     if (ii < nb && j < nb) {
       const int64_t o = p * nb * nb + ii * nb + j;
       Bm[o] = c.at(r);
-      A[o] = ii >= j ? cconj(Rp[j * nb + ii]) : czero();
+      A[o] = aij[r];
     }
+  }
+}
+
+// The same for a single tile (nb <= 16): one step of four in k per wave, the
+// four partial products added through LDS.  A wave alone takes its 16 matrix
+// instructions one after another and was slower than a plain sum per entry
+// (64 problems of 3000 rows, 16 bands, whole adjoint: 54.4 us with such sums,
+// 56.2 with one wave, 53.4 so).
+__global__ __launch_bounds__(256) void qr_bwd_tile_kernel(
+    const double2* __restrict__ G, const double2* __restrict__ rinv,
+    double2* __restrict__ A, double2* __restrict__ Bm, int nb) {
+  __shared__ double2 part[3][4][64];
+  const int64_t o = (int64_t)blockIdx.x * nb * nb;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ii = 4 * s + lk;
+  TileAcc c;
+  double2 a, b;
+  adjoint_step(G + o, rinv + o, nb, li, li, ii, a, b);
+  c.step(a, b);
+  if (ii < nb && li < nb) A[o + ii * nb + li] = b;
+  if (s > 0)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[s - 1][r][lane] = c.at(r);
+  __syncthreads();
+  if (s > 0) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const double2 v = cadd(cadd(c.at(r), part[0][r][lane]),
+                           cadd(part[1][r][lane], part[2][r][lane]));
+    if (4 * r + lk < nb && li < nb) Bm[o + (4 * r + lk) * nb + li] = v;
   }
 }
 
 int launch_qr_bwd_small(const double2* G, const double2* rinv, double2* A,
                         double2* Bm, int64_t P, int nb, hipStream_t s) {
   const int T = (nb + 15) / 16;
-  hipLaunchKernelGGL(qr_bwd_small_kernel,
-                     dim3((T * T + 3) / 4, (unsigned)P), dim3(256), 0, s, G,
-                     rinv, A, Bm, nb, T);
+  if (T == 1)
+    hipLaunchKernelGGL(qr_bwd_tile_kernel, dim3((unsigned)P), dim3(256), 0, s,
+                       G, rinv, A, Bm, nb);
+  else
+    hipLaunchKernelGGL(qr_bwd_small_kernel,
+                       dim3((T * T + 3) / 4, (unsigned)P), dim3(256), 0, s, G,
+                       rinv, A, Bm, nb, T);
   JRX_LAUNCH_CHECK();
   return JRX_OK;
 }

@@ -420,7 +420,6 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
     return rc;
   JRX_CHECK_HIP(hipStreamSynchronize(nullptr));
   p->gsw = gram_split(p->P, ng, nb);
-  p->gsq = p->gsw;
   const int64_t kin_gather =
       p->S * (p->rowpath ? p->row_chunks : p->geo.nxa);
   const int64_t kin_plain = p->S * ((ng + kRedBlock - 1) / kRedBlock);
@@ -433,20 +432,29 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
     off = align_up(off + bytes);
     return o;
   };
-  const size_t mat = (size_t)p->P * nb * nb * sizeof(double2);
+  const size_t mat_one = (size_t)nb * nb * sizeof(double2);
+  const size_t mat = p->P * mat_one;
   p->o_q = take((size_t)p->S * ng * sizeof(double2));
   p->o_qbar = take((size_t)p->S * ng * sizeof(double2));
-  p->o_T = take((size_t)p->chunk * per_state);
   p->o_rho = take((size_t)p->ns * p->N * sizeof(double));
+  // The buffers of the density and adjoint sweeps and of the potential stage
+  // are dead while a Gram matrix is formed: its partial sums share their
+  // place.
+  const size_t sweeps = off;
+  p->o_T = take((size_t)p->chunk * per_state);
   p->o_rpart = take((size_t)p->groups * p->N * sizeof(double));
   p->o_v = take((size_t)p->ns * p->N * sizeof(double));
   p->o_box = take((size_t)p->N * sizeof(double2));
+  auto part_bytes = [&] { return p->P * p->gsw.nchunk * mat_one; };
+  if (part_bytes() > off - sweeps) p->gsw = gram_split(p->P, ng, nb, kQrRows);
+  p->gsq = p->gsw;
+  p->o_part = sweeps;
+  if (part_bytes() > off - sweeps) off = align_up(sweeps + part_bytes());
   p->o_S = take(mat);
   p->o_R1 = take(mat);
   p->o_Ri = take(mat);
   p->o_A = take(mat);
   p->o_Bm = take(mat);
-  p->o_part = take((size_t)p->P * p->gsw.nchunk * nb * nb * sizeof(double2));
   p->o_kin = take((size_t)p->kin_parts_max * sizeof(double));
   p->o_tb = take((size_t)p->S * sizeof(double));
   p->o_eh = take((size_t)p->rec_parts * sizeof(double));

@@ -18,7 +18,7 @@
 
 namespace jrx {
 
-GramSplit gram_split(int64_t P, int ng, int nb) {
+GramSplit gram_split(int64_t P, int ng, int nb, int unit) {
   const int tiles = (ng + kQrRows - 1) / kQrRows;
   // about 2048 blocks in all; the wide kernels do four to sixteen times
   // the work per row, and each chunk adds an nb x nb partial to reduce
@@ -28,7 +28,7 @@ GramSplit gram_split(int64_t P, int ng, int nb) {
   if (want > tiles) want = tiles;
   // whole 64-row tiles; for the wide kernels whole 16-row slabs, so that one
   // block a CU leaves no CU without (137 059 rows: 252 blocks instead of 238)
-  const int unit = nb > kNarrowBands ? 16 : kQrRows;
+  if (unit <= 0) unit = nb > kNarrowBands ? 16 : kQrRows;
   const int units = (ng + unit - 1) / unit;
   GramSplit sp;
   sp.rows_per_chunk = (int)((units + want - 1) / want) * unit;

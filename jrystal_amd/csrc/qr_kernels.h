@@ -22,7 +22,9 @@ struct GramSplit {
   int rows_per_chunk;  // multiple of kQrRows (wide kernels: of 16)
   int nchunk;          // chunks per problem
 };
-GramSplit gram_split(int64_t P, int ng, int nb);
+// unit: rows the chunks are whole multiples of (0: by the band count; kQrRows
+// makes fewer chunks of the wide kernels, hence fewer partials).
+GramSplit gram_split(int64_t P, int ng, int nb, int unit = 0);
 
 // Largest LDS allocation (bytes per workgroup) of the QR kernels for nb.
 size_t qr_lds_bytes(int nb);

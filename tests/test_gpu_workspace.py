@@ -1,0 +1,51 @@
+"""Workspace of plans of more than 64 bands: the partial Gram sums share the
+place of the sweep buffers, so that no plan needs more than with 64-row Gram
+chunks beside them (the totals below) and what fitted the static workspace
+still does."""
+import numpy as np
+import pytest
+import torch
+
+from jrystal_amd import _lib
+from jrystal_amd.objective import EnergyPlan
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(chunk):
+  f = np.arange(24)
+  f = np.where(f < 12, f, f - 24)
+  mask = f[:, None, None]**2 + f[:, None]**2 + f**2 <= 100
+  kpts = np.linspace(0.0, 0.2, 12).reshape(4, 3)
+  occ = np.linspace(2.0, 1.0, 264).reshape(1, 4, 66)
+  return EnergyPlan(np.zeros((1, 3)), np.array([4.0]), 7.0 * np.eye(3), mask,
+                    kpts, occ, chunk_states=chunk)
+
+
+def test_wide_bands_within_the_static_workspace():
+  # 1 and 32 states a chunk: the sweep buffers do not hold 53 Gram chunks a
+  # problem, so 33, which they hold at 32; 60: 53
+  former = {1: 47506176, 32: 56934144, 60: 62353152}
+  gen = torch.Generator(device="cuda").manual_seed(0)
+  w, ref = None, None
+  L = _lib.lib()
+  for chunk, most in former.items():
+    plan = _plan(chunk)
+    assert plan.workspace_bytes <= most <= _lib.STATIC_WORKSPACE_BYTES
+    if w is None:
+      w = [torch.randn(plan.param_shape, generator=gen, device="cuda",
+                       dtype=torch.float64) for _ in range(2)]
+    r = plan.evaluate(*w, grad=True)
+    a = [r[k] for k in ("energies", "dw_re", "dw_im")]
+    b = [torch.full_like(x, np.nan) for x in a]
+    _lib.check(L.jrx_energy_grad_static(
+      plan._plan, w[0].data_ptr(), w[1].data_ptr(),
+      *(x.data_ptr() for x in b), None, None, _lib.stream_ptr()))
+    for x, y in zip(a, b):
+      assert torch.equal(x, y)
+    ref = ref or a
+    # sums in another order: a few rounding errors, amplified by the
+    # condition number of a random W (below 10)
+    for x, y in zip(a, ref):
+      assert torch.linalg.norm(x - y) <= 2e-13 * torch.linalg.norm(y)
+    plan.close()

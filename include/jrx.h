@@ -132,7 +132,7 @@ int jrx_energy_grad(jrx_plan* plan, const double* w_re, const double* w_im,
  * nothing; the plan itself is still made by jrx_plan_create.  Plans whose
  * jrx_plan_workspace_bytes exceeds the limit are rejected with
  * JRX_ERR_UNSUPPORTED (the 2-atom 32^3 / 8 k / 8-band cell needs about
- * 23 MB).  Every call on one GPU shares that GPU's array: calls that overlap
+ * 14 MB).  Every call on one GPU shares that GPU's array: calls that overlap
  * on one GPU (two streams, two host threads) race, and the array keeps the
  * last call's contents, so the plan-level readers of a workspace
  * (jrx_plan_band_norms, jrx_plan_precondition, ...) do not apply to it.
@@ -355,7 +355,10 @@ int jrx_vec_axpby(double alpha, const double* x, double beta, const double* y,
  * ---------------------------------------------------------------------- */
 /* unitary_module.unitary_matrix (unitary_module.py:30-81) for P problems:
  * q [P][nb][ng] (band-major) orthonormal columns of W = w_re + i w_im
- * ([P][ng][nb]); rinv [P][nb][nb] = R^-1 (upper), kept for the backward. */
+ * ([P][ng][nb]); rinv [P][nb][nb] = R^-1 (upper), kept for the backward.
+ * jrx_qr_workspace_bytes is the size for the fastest split of the Gram sums;
+ * with more than 64 bands a coarser one is taken in a workspace that holds
+ * only that. */
 size_t jrx_qr_workspace_bytes(int64_t P, int ng, int nb);
 int jrx_qr(const double* w_re, const double* w_im, int64_t P, int ng, int nb,
            double* q, double* rinv, void* workspace, size_t workspace_bytes,

@@ -673,26 +673,35 @@ int jrx_ewald(const double* positions, const double* charges, int natom,
 }
 
 // ------------------------------------------------------ stand-alone QR --
-static size_t qr_ws_layout(int64_t P, int ng, int nb, size_t* o_part,
-                           size_t* o_s, size_t* o_a, size_t* o_b) {
-  const GramSplit sp = gram_split(P, ng, nb);
-  const size_t mat = (size_t)P * nb * nb * sizeof(double2);
-  size_t off = 0;
-  auto take = [&](size_t b) {
-    size_t o = off;
-    off = (off + b + 255) & ~(size_t)255;
-    return o;
-  };
-  *o_part = take((size_t)P * sp.nchunk * nb * nb * sizeof(double2));
-  *o_s = take(mat);
-  *o_a = take(mat);
-  *o_b = take(mat);
-  return off;
+// Partial Gram sums, the Gram matrix and R1^-1; the adjoint's two factors,
+// formed when its partial sums are added up, take the place of those.
+struct QrLayout {
+  GramSplit split;
+  size_t o_part, o_s, o_r, bytes;
+  QrLayout(int64_t P, int ng, int nb, int unit = 0)
+      : split(gram_split(P, ng, nb, unit)) {
+    const size_t mat = (size_t)P * nb * nb * sizeof(double2);
+    size_t off = 0;
+    auto take = [&](size_t b) {
+      size_t o = off;
+      off = (off + b + 255) & ~(size_t)255;
+      return o;
+    };
+    o_part = take((split.nchunk > 2 ? split.nchunk : 2) * mat);
+    o_s = take(mat);
+    o_r = take(mat);
+    bytes = off;
+  }
+};
+// The layout for a workspace of so many bytes: chunks of whole 64-row tiles
+// where the finer ones of many bands do not fit.
+static QrLayout qr_layout(int64_t P, int ng, int nb, size_t workspace_bytes) {
+  const QrLayout l(P, ng, nb);
+  return l.bytes <= workspace_bytes ? l : QrLayout(P, ng, nb, kQrRows);
 }
 
 size_t jrx_qr_workspace_bytes(int64_t P, int ng, int nb) {
-  size_t a, b, c, d;
-  return qr_ws_layout(P, ng, nb, &a, &b, &c, &d);
+  return QrLayout(P, ng, nb).bytes;
 }
 
 int jrx_qr(const double* w_re, const double* w_im, int64_t P, int ng, int nb,
@@ -706,15 +715,14 @@ int jrx_qr(const double* w_re, const double* w_im, int64_t P, int ng, int nb,
     set_error("nb above 128 is not supported by this build");
     return JRX_ERR_UNSUPPORTED;
   }
-  size_t op, os, oa, ob;
-  const size_t need = qr_ws_layout(P, ng, nb, &op, &os, &oa, &ob);
-  JRX_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace & 255) == 0,
+  const QrLayout l = qr_layout(P, ng, nb, workspace_bytes);
+  JRX_REQUIRE(workspace_bytes >= l.bytes && ((uintptr_t)workspace & 255) == 0,
               "qr workspace too small or misaligned");
   char* ws = (char*)workspace;
-  double2* part = (double2*)(ws + op);
-  double2* S = (double2*)(ws + os);
-  double2* R1 = (double2*)(ws + oa);
-  const GramSplit sp = gram_split(P, ng, nb);
+  double2* part = (double2*)(ws + l.o_part);
+  double2* S = (double2*)(ws + l.o_s);
+  double2* R1 = (double2*)(ws + l.o_r);
+  const GramSplit& sp = l.split;
   hipStream_t s = (hipStream_t)stream;
   int rc;
   if ((rc = launch_gram_gmajor(w_re, w_im, nullptr, part, P, ng, nb, sp, s)) ||
@@ -742,16 +750,15 @@ int jrx_qr_backward(const double* q, const double* qbar, const double* rinv,
     set_error("nb above 128 is not supported by this build");
     return JRX_ERR_UNSUPPORTED;
   }
-  size_t op, os, oa, ob;
-  const size_t need = qr_ws_layout(P, ng, nb, &op, &os, &oa, &ob);
-  JRX_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace & 255) == 0,
+  const QrLayout l = qr_layout(P, ng, nb, workspace_bytes);
+  JRX_REQUIRE(workspace_bytes >= l.bytes && ((uintptr_t)workspace & 255) == 0,
               "qr workspace too small or misaligned");
   char* ws = (char*)workspace;
-  double2* part = (double2*)(ws + op);
-  double2* G = (double2*)(ws + os);
-  double2* A = (double2*)(ws + oa);
-  double2* Bm = (double2*)(ws + ob);
-  const GramSplit sp = gram_split(P, ng, nb);
+  double2* part = (double2*)(ws + l.o_part);
+  double2* G = (double2*)(ws + l.o_s);
+  double2* A = part;
+  double2* Bm = part + P * nb * nb;
+  const GramSplit& sp = l.split;
   hipStream_t s = (hipStream_t)stream;
   int rc;
   if ((rc = launch_gram_bmajor((const double2*)q, (const double2*)qbar, part,

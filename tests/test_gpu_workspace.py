@@ -1,12 +1,12 @@
-"""Workspace of plans of more than 64 bands: the partial Gram sums share the
+"""Workspace of more than 64 bands.  Plans: the partial Gram sums share the
 place of the sweep buffers, so that no plan needs more than with 64-row Gram
 chunks beside them (the totals below) and what fitted the static workspace
-still does."""
+still does.  Stand-alone QR: a workspace for 64-row chunks is enough."""
 import numpy as np
 import pytest
 import torch
 
-from jrystal_amd import _lib
+from jrystal_amd import _lib, _ops
 from jrystal_amd.objective import EnergyPlan
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +49,37 @@ def test_wide_bands_within_the_static_workspace():
     for x, y in zip(a, ref):
       assert torch.linalg.norm(x - y) <= 2e-13 * torch.linalg.norm(y)
     plan.close()
+
+
+@pytest.mark.parametrize("P,ng,nb", [(4, 4169, 66), (1, 17000, 128),
+                                     (3, 150, 80), (2, 60, 16)])
+def test_qr_in_a_workspace_of_64_row_chunks(P, ng, nb):
+  tiles = -(-ng // 64)
+  want = min(-(-(256 if nb > 64 else 2048) // P), tiles)
+  chunks = -(-tiles // -(-tiles // want))
+  former = (chunks + 3) * P * nb * nb * 16 + 4 * 256
+  L = _lib.lib()
+  gen = torch.Generator(device="cuda").manual_seed(nb)
+  new = lambda *s, t=torch.float64: torch.randn(  # noqa: E731
+    s, generator=gen, device="cuda", dtype=t)
+  w, qb = [new(P, ng, nb) for _ in range(2)], new(P, nb, ng,
+                                                  t=torch.complex128)
+  res = []
+  for nbytes in (max(former, L.jrx_qr_workspace_bytes(P, ng, nb)), former):
+    buf, ws = _ops.workspace(nbytes)
+    q = torch.empty((P, nb, ng), dtype=torch.complex128, device="cuda")
+    ri = torch.empty((P, nb, nb), dtype=torch.complex128, device="cuda")
+    g = [torch.empty_like(x) for x in w]
+    s = _lib.stream_ptr()
+    _lib.check(L.jrx_qr(w[0].data_ptr(), w[1].data_ptr(), P, ng, nb,
+                        q.data_ptr(), ri.data_ptr(), ws, nbytes, s))
+    _lib.check(L.jrx_qr_backward(q.data_ptr(), qb.data_ptr(), ri.data_ptr(),
+                                 P, ng, nb, g[0].data_ptr(), g[1].data_ptr(),
+                                 ws, nbytes, s))
+    res.append([q, ri, *g])
+    with pytest.raises(ValueError, match="workspace"):
+      _lib.check(L.jrx_qr(w[0].data_ptr(), w[1].data_ptr(), P, ng, nb,
+                          q.data_ptr(), ri.data_ptr(), ws, 3 * 256, s))
+  for a, b in zip(*res):  # rounding errors of differently grouped sums,
+    # amplified by the condition number (up to 30 at 60 or 150 rows)
+    assert torch.linalg.norm(a - b) <= 1e-12 * torch.linalg.norm(b)

@@ -22,7 +22,8 @@
 namespace jrx {
 
 // Lengths with an alias-free window (PR 1) only; 32, 64 and 128 also have the
-// tighter one (PR 2), 64 and 128 kernels for any mask (PR 0).
+// tighter one (PR 2), 64 the wider one (PR 3), 64 and 128 kernels for any
+// mask (PR 0).
 #define JRX_Z_SIZES(X)                                                      \
   X(35) X(36) X(40) X(42) X(45) X(48) X(49) X(50) X(54) X(56) X(60) X(63)   \
   X(70) X(72) X(75) X(80)
@@ -37,7 +38,7 @@ static int window_of(int n, int m, bool row) {
     case 32:
       return tight ? 2 : fits ? 1 : -1;
     case 64:
-      return tight ? 2 : fits ? 1 : 0;
+      return tight ? 2 : fits ? 1 : m <= 3 * n / 8 - 1 ? 3 : 0;
     case 128:
       return tight ? 2 : 0;
 #define JRX_X(NN) case NN:
@@ -83,6 +84,7 @@ static int unsupported_box() {
   case 64 * 4 + 0: return CALL(64, 0);                                      \
   case 64 * 4 + 1: return CALL(64, 1);                                      \
   case 64 * 4 + 2: return CALL(64, 2);                                      \
+  case 64 * 4 + 3: return CALL(64, 3);                                      \
   case 128 * 4 + 0: return CALL(128, 0);                                    \
   case 128 * 4 + 2: return CALL(128, 2);
 #define JRX_Z_DISPATCH(CALL)                                                \
@@ -153,9 +155,11 @@ static int zplane_groups(const BoxGeom& geo, int nstates,
 // the times at 22 sizes of 32 to 80 points and 64 to 1984 states, every G up
 // to 2304 blocks; on average within 2.2 % (density) and 1.4 % (vpsi) of the
 // best G.  8 waves a block (128 points, wide masks of 64) fill a CU by one
-// block, two in the density pass of 64 points: then as few blocks as keep
-// the CUs full are best (128^3, 128 states, density: 545 us with 2 groups,
-// 575 with 8, 621 with 16), and no tail shows.
+// block; then as few blocks as keep the CUs full are best (128^3, 128 states,
+// density: 545 us with 2 groups, 575 with 8, 621 with 16), and no tail shows.
+// Two such blocks share a CU in the density pass of 64 points and in its v psi
+// pass with a window: at 2048 states of |m| <= 17 the latter takes 2650 us
+// with one block a CU (4 groups), 2040 with 8, 1970 with 16 and 1900 with 32.
 static bool wide_blocks(const BoxGeom& geo) {
   return geo.nx == 128 || (geo.nx == 64 && z_window(geo) != 2);
 }
@@ -175,9 +179,12 @@ int zplane_density_groups(const BoxGeom& geo, int nstates) {
                             : GroupWeights{most, 1, 0.25, 0.4});
 }
 int zplane_vpsi_groups(const BoxGeom& geo, int nstates) {
+  if (!wide_blocks(geo))
+    return zplane_groups(geo, nstates, GroupWeights{3072, 1, 1.5, 0.4});
+  const bool two = geo.nx == 64 && z_window(geo) != 0;
   return zplane_groups(geo, nstates,
-                       wide_blocks(geo) ? GroupWeights{2048, 1, 0.0, 0.3}
-                                        : GroupWeights{3072, 1, 1.5, 0.4});
+                       two ? GroupWeights{2048, 2, 0.3, 0.4}
+                           : GroupWeights{2048, 1, 0.0, 0.3});
 }
 
 int launch_row_ifft(const double2* q, double2* R, int64_t state0, int nstates,

@@ -2,8 +2,9 @@
 // N of the z axis, and z-plane passes, one set per side N of the square (x, y)
 // planes; each with the mask's window PR along the axes it transforms:
 //   PR 1: every mask point has |m| <= N / 4 (a density box that is free of
-//         aliasing); PR 2: |m| <= N / 4 - 1; PR 0: any mask (z-plane passes:
-//         of at most 64 x-planes; N = 64 and 128 only).
+//         aliasing); PR 2: |m| <= N / 4 - 1; PR 3: |m| <= 3 N / 8 - 1 (N = 64
+//         only); PR 0: any mask (z-plane passes: of at most 64 x-planes;
+//         N = 64 and 128 only).
 // With a window, the first radix stage of an inverse transform has about half
 // of its inputs and the last one of a forward transform about half of its
 // outputs: the loads, stores and additions of the rest are not there.
@@ -86,7 +87,9 @@ JRX_ZSHAPE(128, 8, 8, 0, 0, 0)
 template <int N, int PR>
 struct Window {
   static constexpr int V = RegLine<N>::V, L = RegLine<N>::L;
-  static constexpr int Q = PR == 2 ? N / 4 - 1 : N / 4;
+  static constexpr int Q = PR == 3   ? 3 * N / 8 - 1
+                           : PR == 2 ? N / 4 - 1
+                                     : N / 4;
   static constexpr int LO = PR ? (Q + L) / L : V;  // ceil((Q + 1) / L)
   static constexpr int HI = PR ? (Q + L - 1) / L : 0;
   static constexpr int M = LO + HI;
@@ -567,7 +570,11 @@ int RowPass<N, PR>::gather(const double2* R, const double2* q, double2* qbar,
 }
 
 // 64-point masks of 33 or more x-planes: 512 threads, so that one column
-// pass is enough.
+// pass is enough.  With a window v psi then fits 128 registers without the
+// prefetch, and two blocks share a CU; any mask takes 132 without it, so
+// the next state's inputs are prefetched instead (180).  v psi of 2048
+// states: |m| <= 17, PR 0 without prefetch 2650 us, with it 2310, PR 3 1900
+// (with prefetch 2310); |m| <= 28, PR 0 without prefetch 3400, with it 2650.
 template <int N, int PR>
 struct ZWide {
   static constexpr bool value = N == 64 && PR != 2;
@@ -580,7 +587,7 @@ int ZPass<N, PR>::density(const double2* R, double* rho_part, int groups,
                             const double2* tw, bool store, hipStream_t s) {
   using S = ZShape<N>;
   constexpr int NW = ZWide<N, PR>::value ? 8 : S::NWD;
-  constexpr bool PF = PR != 0 && S::PFD;
+  constexpr bool PF = PR != 0 && PR != 3 && S::PFD;
   hipLaunchKernelGGL((zplane_density_kernel<N, PR, NW, PF>),
                      dim3(geo.nz, groups), dim3(NW * 64),
                      (ZPlane<N, PR, NW>::kLds), s, R, rho_part, occ, state0,
@@ -594,8 +601,9 @@ int ZPass<N, PR>::vpsi(double2* R, const double* v, int groups, int nstates,
                          const BoxGeom& geo, const double2* tw,
                          hipStream_t s) {
   using S = ZShape<N>;
-  constexpr int NW = ZWide<N, PR>::value ? 8 : S::NW;
-  constexpr bool VR = S::VR, PF = PR != 0 && S::PFV;
+  constexpr bool wide = ZWide<N, PR>::value;
+  constexpr int NW = wide ? 8 : S::NW;
+  constexpr bool VR = S::VR, PF = wide ? PR == 0 : PR != 0 && S::PFV;
   hipLaunchKernelGGL((zplane_vpsi_kernel<N, PR, NW, VR, PF>),
                      dim3(geo.nz, groups), dim3(NW * 64),
                      (ZPlane<N, PR, NW>::kLds), s, R, v, nstates, geo, tw);

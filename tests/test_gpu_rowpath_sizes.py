@@ -173,3 +173,26 @@ def test_last_chunk_with_more_groups(n, nb, chunk):
   assert path
   _, b = _run(n, mask, 1, nb, band=True, fft_variant=1)
   _close(a, b)
+
+
+@pytest.mark.parametrize("q", (17, 22, 23, 24, 31))
+@pytest.mark.parametrize("nb", (3, 40))
+def test_row_path_64_masks_beyond_the_alias_free_window(q, nb):
+  """The wider window (|m| <= 23) and no window, along x and y and along z
+  alone, with one state and several states a group."""
+  for qxy, qz in ((q, 15), (15, q), (q, q)):
+    mask = _mask(64, qxy, qz=qz)
+    path, a = _run(64, mask, 1, nb, band=True)
+    assert path
+    _, b = _run(64, mask, 1, nb, band=True, fft_variant=1)
+    _close(a, b)
+
+
+@pytest.mark.parametrize("n,nz", ((32, 64), (64, 48)))
+def test_long_boxes_with_the_wider_window_of_64(n, nz):
+  mask = _mask(n, 23 if n == 64 else 8, 0.2, seed=1, nz=nz,
+               qz=23 if nz == 64 else 12)
+  path, a = _run(n, mask, 2, 2, band=True)
+  assert path
+  _, b = _run(n, mask, 2, 2, band=True, fft_variant=1)
+  _close(a, b)

@@ -6,14 +6,17 @@ fastest:
 * FFT variant: the compile-time-radix kernels where they exist (64^3
   uses the register-resident 64-point kernels) or the runtime-radix ones;
 * x-line workgroup target: how many state groups the x-line passes split
-  the states into (2048, 4096 or 8192 workgroups);
+  the states into (2048, 4096 or 8192 workgroups; plans on the row path have
+  no x-line pass and are not timed again for it);
 * state chunking: all states in one chunk (forward planes kept for the
   adjoint sweep) or half / a quarter of them per chunk.
 
 Every variant computes the same energy and gradient; only the schedule
 changes.  Results are cached in a JSON file keyed by the shape (grid,
-G-sphere size, spins, k-points, bands).
+G-sphere size, spins, k-points, bands), each with the digest of the library
+it was timed with: another build times the shape again.
 """
+import hashlib
 import json
 import os
 import time
@@ -21,6 +24,7 @@ import time
 import numpy as np
 import torch
 
+from . import _lib
 from .objective import EnergyPlan
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "jrystal_amd",
@@ -59,6 +63,12 @@ def _time(plan, w_re, w_im, reps):
   return (time.perf_counter() - t0) / reps
 
 
+def library_digest() -> str:
+  """Digest of the built library's file."""
+  with open(_lib.LIB_PATH, "rb") as f:
+    return hashlib.sha256(f.read()).hexdigest()[:16]
+
+
 def tune(wl, cache_path: str = DEFAULT_CACHE, reps: int = 3, device=None,
          refresh: bool = False, log=None):
   """Fastest plan options for wl's shape (cached)."""
@@ -70,22 +80,28 @@ def tune(wl, cache_path: str = DEFAULT_CACHE, reps: int = 3, device=None,
         cache = json.load(f)
     except (OSError, ValueError):
       cache = {}
-  if key in cache:
+  build = library_digest()
+  if key in cache and cache[key].get("library") == build:
     return dict(cache[key]["options"])
   p = wl.params(0)
   dev = torch.device(device if device is not None else "cuda")
   w_re = torch.tensor(p["w_re"], device=dev)
   w_im = torch.tensor(p["w_im"], device=dev)
   results = []
+  row_path = False
   for opt in candidates(wl):
+    if row_path and opt["xline_blocks"]:
+      continue
     plan = EnergyPlan.from_workload(wl, device=dev, **opt)
+    if opt == candidates_default():
+      row_path = plan.row_path
     t = _time(plan, w_re, w_im, reps)
     plan.close()
     results.append((t, opt))
     if log:
       log(f"autotune {key} {opt}: {t * 1e3:.3f} ms")
   t_best, best = min(results, key=lambda r: r[0])
-  cache[key] = {"options": best, "ms": t_best * 1e3,
+  cache[key] = {"options": best, "ms": t_best * 1e3, "library": build,
                 "tried": [{"options": o, "ms": t * 1e3} for t, o in results]}
   if cache_path:
     os.makedirs(os.path.dirname(cache_path), exist_ok=True)

@@ -1,12 +1,12 @@
 // Register transforms of one line of N points on L lanes of a wavefront.
 //
-// N = V * L.  Lane j of a line holds x[j + L m] in v[m] (m < V).  to_ab runs a V-point DFT over m in registers, multiplies by w_N^{ja},
-// transposes blocks of L registers over the L lanes, and runs W = ceil(V / L)
-// L-point DFTs: lane i ends with X[a + V b] in v[u L + b], a = i + L u
-// (u < W; where a >= V the lane holds nothing of use).  The forward transform
-// is its mirror image, so a product with v(r) between the two needs no
-// further exchange.  64 / L lines share a wave and never leave it: no block
-// barrier inside.
+// N = V * L.  Lane j of a line holds x[j + L m] in v[m] (m < V).  to_ab runs a
+// V-point DFT over m in registers, multiplies by w_N^{ja}, transposes blocks
+// of L registers over the L lanes, and runs W = ceil(V / L) L-point DFTs: lane
+// i ends with X[a + V b] in v[u L + b], a = i + L u (u < W; where a >= V the
+// lane holds nothing of use).  The forward transform is its mirror image, so a
+// product with v(r) between the two needs no further exchange.  64 / L lines
+// share a wave and never leave it: no block barrier inside.
 //
 // The transposition is what such a transform costs beside its arithmetic.
 // Measured on gfx950 (cycles of a CU per wave access, conflict-free): a
@@ -15,15 +15,16 @@
 // arithmetic takes on the four SIMDs.  With L = 4, the lanes of a line 16
 // apart, it is two v_permlane*_swap per register pair instead (32 VALU
 // instructions for eight values, no LDS); with L = 8, lanes 8 apart, a third
-// stage by row rotation.  Sizes that 4 does not divide exchange through LDS.
+// stage by row rotation.  The other L exchange through LDS.
 //
 // The small DFTs are written with compile-time constants: powers of two by
 // radix 2 / 4 / 8, odd primes by the symmetric sums u_k +- u_{p-k} (half the
 // products of the direct sum), coprime products by index maps without
 // twiddles (Good 1958), 9 and 16 by one Cooley-Tukey step.  Inputs that are
 // literal zeros (the part of the box outside the mask's window) and outputs
-// that nobody reads fold away; the files that include this are built with
-// -fno-signed-zeros, without which x + 0 stays an addition.
+// that nobody reads fold away; the files of the row-path kernels
+// (rowfft_*.hip) are built with -fno-signed-zeros, without which x + 0 stays
+// an addition.  (The full-box kernels have no zero inputs.)
 #pragma once
 #include "fft_core.h"
 

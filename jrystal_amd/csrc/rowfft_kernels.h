@@ -53,7 +53,12 @@ struct RowBlock {
 // fastest of the sets measured at 432 states of an alias-free cubic box
 // (time per state and box point, density / v psi: 2.9 / 4.0 ps at 32, 2.9 /
 // 5.1 at 45, 2.5 / 3.8 at 48, 1.9 / 3.1 at 64, 2.7 / 4.9 at 75); a set that
-// spills registers loses up to a factor of two.
+// spills many registers loses up to a factor of two.  Kernels that spill a few
+// and are still the fastest measured: v psi of 42 points (4 registers; 1984
+// states 639 us, without the prefetch and the spill 674) and the 128-point
+// kernels without a window (density 24, v psi 4; 512 states of |m| <= 40:
+// 2530 and 4500 us, and 4030 and 4490 with the y lines split over two blocks
+// and LDS exchange).
 template <int N>
 struct ZShape;
 #define JRX_ZSHAPE(NN, NW_, NWD_, VR_, PFV_, PFD_)                       \

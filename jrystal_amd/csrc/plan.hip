@@ -3,6 +3,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
@@ -239,6 +240,7 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   std::vector<int> plane_g0, plane_x, g_yz, row_off, row_g0, g_row;
   std::vector<short> rows, g_m;
   int ng = 0, max_rows = 0;
+  int most_xy = 0, most_z = 0;  // largest |integer frequency| of a mask point
   auto fq = [](int j, int n) { return j < (n + 1) / 2 ? j : j - n; };
   for (int x = 0; x < nx; ++x) {
     int first = -1;
@@ -253,14 +255,20 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
           g_yz.push_back(y * nz + z);
           g_m.push_back((short)fq(x, nx));
           g_m.push_back((short)fq(y, ny));
-          g_m.push_back((short)fq(z, nz));
+          const int mz = fq(z, nz);
+          most_z = std::max(most_z, abs(mz));
+          g_m.push_back((short)mz);
           ++ng;
           any = true;
         }
       }
-      if (any) prow.push_back((short)y);
+      if (any) {
+        prow.push_back((short)y);
+        most_xy = std::max(most_xy, abs(fq(y, ny)));
+      }
     }
     if (first >= 0) {
+      most_xy = std::max(most_xy, abs(fq(x, nx)));
       plane_g0.push_back(first);
       plane_x.push_back(x);
       row_off.push_back((int)rows.size());
@@ -285,11 +293,8 @@ int plan_build(jrx_plan* p, const jrx_problem* d) {
   p->geo.nx = nx; p->geo.ny = ny; p->geo.nz = nz; p->geo.ng = ng;
   p->geo.nxa = (int)plane_x.size();
   p->geo.max_rows = max_rows;
-  p->geo.mmax_xy = p->geo.mmax_z = 0;
-  for (size_t i = 0; i < g_m.size(); ++i) {
-    int& most = i % 3 == 2 ? p->geo.mmax_z : p->geo.mmax_xy;
-    if (abs(g_m[i]) > most) most = abs(g_m[i]);
-  }
+  p->geo.mmax_xy = most_xy;
+  p->geo.mmax_z = most_z;
   int rc;
   int* tmp = nullptr;
   if ((rc = upload(p, plane_g0.data(), plane_g0.size(), &tmp))) return rc;
